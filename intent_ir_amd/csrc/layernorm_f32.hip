@@ -8,14 +8,19 @@
 // below are compiled with contraction off), so y differs from numpy's only through the order
 // in which the two row sums are accumulated.
 //
-// Three forms, all reading x from HBM once where the row fits in registers:
-//  * N % 4 == 0, N <= 4096, 16-byte aligned tensors: a wave per row, the row held in
-//    registers (kVpl 16-byte vectors per lane), 4 rows per 256-thread workgroup with w and b
-//    staged in LDS once per workgroup (instead of once per row from L2);
-//  * N % 4 == 0, 4096 < N <= 65536, aligned: kW waves per row (the row in registers across
-//    them), the wave sums exchanged through LDS and folded in a fixed order, w and b from L2;
-//  * any other shape (odd N, unaligned views, N > 65536): a 256-thread workgroup per row that
+// Forms, the first two reading x from HBM once with the row held in registers:
+//  * N <= 4099: a wave per row (kVpl 16-byte vectors per lane), 4 rows per 256-thread workgroup
+//    with w and b staged in LDS once per workgroup (instead of once per row from L2);
+//  * 4099 < N <= 65539: kW waves per row, the wave sums exchanged through LDS and folded in a
+//    fixed order, w and b from L2;
+//    both come twice: kU = false for N % 4 == 0 and 16-byte aligned tensors; kU = true for rows
+//    that start at any 4-byte boundary (odd N, unaligned views): the same 16-byte accesses, of
+//    which gfx950 asks 4-byte alignment only, from the row's own start, and the last N % 4
+//    elements on the row's first lanes;
+//  * longer rows, and bases that are not 4-byte aligned: a 256-thread workgroup per row that
 //    reads x three times (the second and third reads of a row come from L2).
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace ihip {
@@ -26,29 +31,61 @@ namespace ihip {
 // (45.7 against 46.8 us, graph replays, rotated buffers) and of 2 or 8.
 constexpr int kLn32Rows = 4;
 
-template <int kVpl>
+// A 16-byte vector of a row, streamed past the caches: 16-byte aligned, or (kU) at any 4-byte
+// boundary.  At [8192, 4099] the kU form runs 52.4 us (5.13 TB/s; 47.9 aligned at N = 4096, and
+// 107.9 for the three-pass form that these rows took before); through the caches, which could
+// merge the lines that neighbouring stores and rows share, its loads and stores took 54.1, its
+// stores alone 52.1, and at [4096, 8195] 56.7 streamed against 61.2 and 58.1.
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+template <bool kU>
+using ln32_vec = std::conditional_t<kU, f32x4_u, f32x4>;
+
+template <bool kU>
+__device__ __forceinline__ f32x4 ln32_load(const float* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const ln32_vec<kU>*>(p));
+}
+template <bool kU>
+__device__ __forceinline__ f32x4 ln32_load_wb(const float* p) {
+  return *reinterpret_cast<const ln32_vec<kU>*>(p);
+}
+template <bool kU>
+__device__ __forceinline__ void ln32_store(float* p, f32x4 v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<ln32_vec<kU>*>(p));
+}
+
+// n4 = N / 4 whole vectors per row; kU: the N % 4 elements after them are on lanes 0..2.
+template <int kVpl, bool kU>
 __global__ __launch_bounds__(64 * kLn32Rows) void layernorm_rows_f32_wave(
-    const f32x4* __restrict__ x, const f32x4* __restrict__ w, const f32x4* __restrict__ b, f32x4* __restrict__ y,
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y,
     float* __restrict__ mean_out, float* __restrict__ rstd_out, int64_t M, int n4, int N, float eps) {
   __shared__ f32x4 w_lds[kVpl * kWave], b_lds[kVpl * kWave];
   const int lane = threadIdx.x & 63;
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * kLn32Rows + (threadIdx.x >> 6);
   const bool live = row0 < M;  // waves past the last row read row M - 1 and store nothing
   const int64_t row = live ? row0 : M - 1;
-  const f32x4* xr = x + row * n4 + lane;
+  const float* xr = x + row * N + 4 * lane;
   f32x4 xv[kVpl];
 #pragma unroll
   for (int i = 0; i < kVpl; ++i)
-    xv[i] = lane + i * kWave < n4 ? __builtin_nontemporal_load(xr + i * kWave) : f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int t = threadIdx.x; t < n4; t += 64 * kLn32Rows) {  // staged after the row loads are issued
-    w_lds[t] = w[t];
-    b_lds[t] = b[t];
+    xv[i] = lane + i * kWave < n4 ? ln32_load<kU>(xr + 4 * i * kWave) : f32x4{0.f, 0.f, 0.f, 0.f};
+  const int te = 4 * n4 + lane;  // this lane's element of the tail
+  const bool tail = kU && te < N;
+  float xt = 0.f, wt = 0.f, bt = 0.f;
+  if (tail) {
+    xt = x[row * N + te];
+    wt = w[te];
+    bt = b[te];
   }
-  float s = 0.f;
+  for (int t = threadIdx.x; t < n4; t += 64 * kLn32Rows) {  // staged after the row loads are issued
+    w_lds[t] = ln32_load_wb<kU>(w + 4 * t);
+    b_lds[t] = ln32_load_wb<kU>(b + 4 * t);
+  }
+  float s = xt;
 #pragma unroll
   for (int i = 0; i < kVpl; ++i) s += (xv[i][0] + xv[i][1]) + (xv[i][2] + xv[i][3]);  // padding holds +0
   const float mean = wave_sum(s) / static_cast<float>(N);
-  float q = 0.f;
+  const float dt = xt - mean;
+  float q = tail ? dt * dt : 0.f;
 #pragma unroll
   for (int i = 0; i < kVpl; ++i) {
     const bool in = lane + i * kWave < n4;
@@ -60,7 +97,7 @@ __global__ __launch_bounds__(64 * kLn32Rows) void layernorm_rows_f32_wave(
   }
   const float rstd = 1.0f / sqrtf(wave_sum(q) / static_cast<float>(N) + eps);
   __syncthreads();  // w and b staged
-  f32x4* yr = y + row * n4;
+  float* yr = y + row * N + 4 * lane;
 #pragma unroll
   for (int i = 0; i < kVpl; ++i) {
     const int idx = lane + i * kWave;  // lanes past n4 read LDS entries never staged and store nothing
@@ -68,8 +105,9 @@ __global__ __launch_bounds__(64 * kLn32Rows) void layernorm_rows_f32_wave(
     f32x4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = ((xv[i][j] - mean) * rstd) * wv[j] + bv[j];
-    if (live && idx < n4) __builtin_nontemporal_store(o, yr + idx);
+    if (live && idx < n4) ln32_store<kU>(yr + 4 * i * kWave, o);
   }
+  if (live && tail) y[row * N + te] = (dt * rstd) * wt + bt;
   if (live && lane == 0) {
     if (mean_out != nullptr) mean_out[row] = mean;
     if (rstd_out != nullptr) rstd_out[row] = rstd;
@@ -77,20 +115,23 @@ __global__ __launch_bounds__(64 * kLn32Rows) void layernorm_rows_f32_wave(
 }
 
 // kW waves per row, one row per workgroup: wave v holds the vectors (v * 64 + lane) + i * 64 * kW.
-template <int kVpl, int kW>
+template <int kVpl, int kW, bool kU>
 __global__ __launch_bounds__(64 * kW) void layernorm_rows_f32_multi(
-    const f32x4* __restrict__ x, const f32x4* __restrict__ w, const f32x4* __restrict__ b, f32x4* __restrict__ y,
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y,
     float* __restrict__ mean_out, float* __restrict__ rstd_out, int n4, int N, float eps) {
   __shared__ float part_s[kW], part_q[kW];
   const int lane = threadIdx.x & 63, v = threadIdx.x >> 6;
   const int64_t row = blockIdx.x;
   const int base = v * kWave + lane;
-  const f32x4* xr = x + row * n4 + base;
+  const float* xr = x + row * N + 4 * base;
   f32x4 xv[kVpl];
 #pragma unroll
   for (int i = 0; i < kVpl; ++i)
-    xv[i] = base + i * kWave * kW < n4 ? __builtin_nontemporal_load(xr + i * kWave * kW) : f32x4{0.f, 0.f, 0.f, 0.f};
-  float s = 0.f;
+    xv[i] = base + i * kWave * kW < n4 ? ln32_load<kU>(xr + 4 * i * kWave * kW) : f32x4{0.f, 0.f, 0.f, 0.f};
+  const int te = 4 * n4 + base;  // this thread's element of the tail
+  const bool tail = kU && te < N;
+  const float xt = tail ? x[row * N + te] : 0.f;
+  float s = xt;
 #pragma unroll
   for (int i = 0; i < kVpl; ++i) s += (xv[i][0] + xv[i][1]) + (xv[i][2] + xv[i][3]);
   s = wave_sum(s);
@@ -100,7 +141,8 @@ __global__ __launch_bounds__(64 * kW) void layernorm_rows_f32_multi(
 #pragma unroll
   for (int k = 0; k < kW; ++k) tot += part_s[k];
   const float mean = tot / static_cast<float>(N);
-  float q = 0.f;
+  const float dt = xt - mean;
+  float q = tail ? dt * dt : 0.f;
 #pragma unroll
   for (int i = 0; i < kVpl; ++i) {
     const bool in = base + i * kWave * kW < n4;
@@ -117,18 +159,19 @@ __global__ __launch_bounds__(64 * kW) void layernorm_rows_f32_multi(
 #pragma unroll
   for (int k = 0; k < kW; ++k) qt += part_q[k];
   const float rstd = 1.0f / sqrtf(qt / static_cast<float>(N) + eps);
-  f32x4* yr = y + row * n4;
+  float* yr = y + row * N + 4 * base;
 #pragma unroll
   for (int i = 0; i < kVpl; ++i) {
     const int idx = base + i * kWave * kW;
     if (idx < n4) {
-      const f32x4 wv = w[idx], bv = b[idx];
+      const f32x4 wv = ln32_load_wb<kU>(w + 4 * idx), bv = ln32_load_wb<kU>(b + 4 * idx);
       f32x4 o;
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[j] = ((xv[i][j] - mean) * rstd) * wv[j] + bv[j];
-      __builtin_nontemporal_store(o, yr + idx);
+      ln32_store<kU>(yr + 4 * i * kWave * kW, o);
     }
   }
+  if (tail) y[row * N + te] = (dt * rstd) * w[te] + b[te];
   if (v == 0 && lane == 0) {
     if (mean_out != nullptr) mean_out[row] = mean;
     if (rstd_out != nullptr) rstd_out[row] = rstd;
@@ -162,51 +205,53 @@ __global__ __launch_bounds__(kLn32AnyThreads) void layernorm_rows_f32_any(
   }
 }
 
-template <int kVpl>
-static void launch_ln32_wave(const f32x4* x4, const f32x4* w4, const f32x4* b4, f32x4* y4, float* mean, float* rstd,
+template <int kVpl, bool kU>
+static void launch_ln32_wave(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
                              int64_t M, int n4, int N, float eps, hipStream_t s) {
   const int64_t blocks = (M + kLn32Rows - 1) / kLn32Rows;
-  layernorm_rows_f32_wave<kVpl><<<dim3(static_cast<unsigned>(blocks)), dim3(64 * kLn32Rows), 0, s>>>(
-      x4, w4, b4, y4, mean, rstd, M, n4, N, eps);
+  layernorm_rows_f32_wave<kVpl, kU><<<dim3(static_cast<unsigned>(blocks)), dim3(64 * kLn32Rows), 0, s>>>(
+      x, w, b, y, mean, rstd, M, n4, N, eps);
 }
 
-template <int kW>
-static void launch_ln32_multi(const f32x4* x4, const f32x4* w4, const f32x4* b4, f32x4* y4, float* mean, float* rstd,
+template <int kW, bool kU>
+static void launch_ln32_multi(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
                               int64_t M, int n4, int N, float eps, hipStream_t s) {
-  layernorm_rows_f32_multi<16, kW><<<dim3(static_cast<unsigned>(M)), dim3(64 * kW), 0, s>>>(x4, w4, b4, y4, mean,
-                                                                                             rstd, n4, N, eps);
+  layernorm_rows_f32_multi<16, kW, kU><<<dim3(static_cast<unsigned>(M)), dim3(64 * kW), 0, s>>>(x, w, b, y, mean, rstd,
+                                                                                               n4, N, eps);
 }
 
-// True when every tensor is 16-byte aligned and rows are whole 16-byte vectors.
-static bool ln32_vector_form(const void* x, const void* w, const void* b, const void* y, int64_t N) {
-  const auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  return N % 4 == 0 && al(x) && al(w) && al(b) && al(y);
+// N / 4 <= 16384 whole vectors per row.
+template <bool kU>
+static void launch_ln32_held(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
+                             int64_t M, int N, float eps, hipStream_t s) {
+  const int n4 = N / 4;
+  if (n4 <= 64) launch_ln32_wave<1, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 128) launch_ln32_wave<2, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 256) launch_ln32_wave<4, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 512) launch_ln32_wave<8, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 1024) launch_ln32_wave<16, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 2048) launch_ln32_multi<2, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 4096) launch_ln32_multi<4, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else if (n4 <= 8192) launch_ln32_multi<8, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  else launch_ln32_multi<16, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+}
+
+// True when every tensor starts at a multiple of `a` bytes.
+static bool ln32_aligned(const void* x, const void* w, const void* b, const void* y, uintptr_t a) {
+  const auto al = [a](const void* p) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
+  return al(x) && al(w) && al(b) && al(y);
 }
 
 hipError_t launch_layernorm_rows_f32(const float* x, const float* w, const float* b, float* y, float* mean,
                                      float* rstd, int64_t M, int64_t N, float eps, hipStream_t s) {
   if (M == 0) return hipSuccess;
   if (M > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (N == 0) {  // mean of an empty row: 0 / 0 (NaN), as numpy's sum / N; y is empty
-    layernorm_rows_f32_any<<<dim3(static_cast<unsigned>(M)), dim3(kLn32AnyThreads), 0, s>>>(x, w, b, y, mean, rstd,
-                                                                                            N, eps);
-    return hipGetLastError();
-  }
-  if (ln32_vector_form(x, w, b, y, N) && N <= 65536) {
-    const auto* x4 = reinterpret_cast<const f32x4*>(x);
-    const auto* w4 = reinterpret_cast<const f32x4*>(w);
-    const auto* b4 = reinterpret_cast<const f32x4*>(b);
-    auto* y4 = reinterpret_cast<f32x4*>(y);
-    const int n4 = static_cast<int>(N / 4), Ni = static_cast<int>(N);
-    if (n4 <= 64) launch_ln32_wave<1>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 128) launch_ln32_wave<2>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 256) launch_ln32_wave<4>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 512) launch_ln32_wave<8>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 1024) launch_ln32_wave<16>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 2048) launch_ln32_multi<2>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 4096) launch_ln32_multi<4>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else if (n4 <= 8192) launch_ln32_multi<8>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
-    else launch_ln32_multi<16>(x4, w4, b4, y4, mean, rstd, M, n4, Ni, eps, s);
+  // N = 0: the mean of an empty row is 0 / 0 (NaN), as numpy's sum / N; y is empty
+  if (N > 0 && N / 4 <= 16384 && ln32_aligned(x, w, b, y, 4)) {
+    if (N % 4 == 0 && ln32_aligned(x, w, b, y, 16))
+      launch_ln32_held<false>(x, w, b, y, mean, rstd, M, static_cast<int>(N), eps, s);
+    else
+      launch_ln32_held<true>(x, w, b, y, mean, rstd, M, static_cast<int>(N), eps, s);
     return hipGetLastError();
   }
   layernorm_rows_f32_any<<<dim3(static_cast<unsigned>(M)), dim3(kLn32AnyThreads), 0, s>>>(x, w, b, y, mean, rstd, N,
