@@ -41,6 +41,8 @@ struct EwJitArgs {
   int64_t shape[4];
   int64_t rows;
   int64_t nvec;  // ceil(D3 / V): lanes own V = 4 or 8 elements
+  // Flat form: all elements as one run, and floor(e / D3) for e < 2^31 as (e * magic) >> shift.
+  uint32_t total, magic, shift;
 };
 
 namespace {
@@ -63,6 +65,7 @@ struct EwJitArgs {
   i64 shape[4];
   i64 rows;
   i64 nvec;
+  u32 total, magic, shift;
 };
 // exp, division and 1/sqrt on the hardware approximations, each refined to within ~2 ulp of
 // the correctly rounded result (the numpy float32 forms the interpreter uses round once or
@@ -205,6 +208,89 @@ template <int DT> __device__ __forceinline__ void st8(void* p, i64 i, const floa
   } else {
     st4<DT>(p, i, v);
     st4<DT>(p, i + 4, v + 4);
+  }
+}
+// EW_V consecutive elements at any element boundary (gfx950 takes vector accesses at any
+// alignment), cached like ld4 / ld8.
+typedef float f32x4_e __attribute__((ext_vector_type(4), aligned(4)));
+typedef u32 u32x4_e4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef u32 u32x4_e2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef u32 u32x2_e2 __attribute__((ext_vector_type(2), aligned(2)));
+typedef u32 u32x2_e1 __attribute__((ext_vector_type(2), aligned(1)));
+typedef u32 u32_e1 __attribute__((aligned(1)));
+template <int DT> __device__ __forceinline__ void ldu(const void* p, i64 i, float* v) {
+  if constexpr (DT == 0) {
+    const f32x4_e q = __builtin_nontemporal_load((const f32x4_e*)((const float*)p + i));
+    for (int j = 0; j < 4; ++j) v[j] = q[j];
+  } else if constexpr (DT == 1 || DT == 2) {
+    u32 w[EW_V / 2];
+    if constexpr (EW_V == 8) {
+      const u32x4_e2 q = *(const u32x4_e2*)((const u16*)p + i);
+      for (int j = 0; j < 4; ++j) w[j] = q[j];
+    } else {
+      const u32x2_e2 q = *(const u32x2_e2*)((const u16*)p + i);
+      for (int j = 0; j < 2; ++j) w[j] = q[j];
+    }
+    for (int j = 0; j < EW_V / 2; ++j) {
+      const u16 lo = (u16)(w[j] & 0xffffu), hi = (u16)(w[j] >> 16);
+      v[2 * j] = DT == 1 ? h2f(lo) : b2f(lo);
+      v[2 * j + 1] = DT == 1 ? h2f(hi) : b2f(hi);
+    }
+  } else if constexpr (DT == 3) {
+    u32 w[EW_V / 4];
+    if constexpr (EW_V == 8) {
+      const u32x2_e1 q = *(const u32x2_e1*)((const u8*)p + i);
+      w[0] = q.x;
+      w[1] = q.y;
+    } else {
+      w[0] = *(const u32_e1*)((const u8*)p + i);
+    }
+    for (int j = 0; j < EW_V; ++j) v[j] = (float)((w[j / 4] >> (8 * (j % 4))) & 0xffu);
+  } else {
+    const u32x4_e4 q = __builtin_nontemporal_load((const u32x4_e4*)((const int*)p + i));
+    for (int j = 0; j < 4; ++j) v[j] = (float)(int)q[j];
+  }
+}
+template <int DT> __device__ __forceinline__ void stu(void* p, i64 i, const float* v) {
+  if constexpr (DT == 0) {
+    __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, (f32x4_e*)((float*)p + i));
+  } else if constexpr (DT == 1 || DT == 2) {
+    if constexpr (EW_V == 8)
+      *(u32x4_e2*)((u16*)p + i) =
+          u32x4{pk2<DT>(v[0], v[1]), pk2<DT>(v[2], v[3]), pk2<DT>(v[4], v[5]), pk2<DT>(v[6], v[7])};
+    else
+      *(u32x2_e2*)((u16*)p + i) = u32x2{pk2<DT>(v[0], v[1]), pk2<DT>(v[2], v[3])};
+  } else if constexpr (DT == 3) {
+    u32 w[EW_V / 4] = {};
+    for (int j = 0; j < EW_V; ++j) w[j / 4] |= (v[j] != 0.0f ? 1u : 0u) << (8 * (j % 4));
+    if constexpr (EW_V == 8)
+      *(u32x2_e1*)((u8*)p + i) = u32x2{w[0], w[1]};
+    else
+      *(u32_e1*)((u8*)p + i) = w[0];
+  } else {
+    __builtin_nontemporal_store(u32x4{(u32)(int)v[0], (u32)(int)v[1], (u32)(int)v[2], (u32)(int)v[3]},
+                                (u32x4_e4*)((int*)p + i));
+  }
+}
+// One operand's EW_V elements in the flat form, for the run of elements starting at e = row * D3
+// + col.  Kinds: 'u' one per element (dense), 'b' one value, and, per column (a bias) or per row
+// of D3 elements: 'x' / 'c' when a run stays inside one row (D3 % EW_V == 0), 'w' / 'd' when it may
+// cross into the next one (D3 >= EW_V), 'W' / 'D' when it may cross several.
+template <int DT, char K> __device__ __forceinline__ void ldf(const void* p, u32 e, u32 row, u32 col, u32 d3, float* v) {
+  if constexpr (K == 'u') {
+    ldu<DT>(p, (i64)e, v);
+  } else if constexpr (K == 'x') {
+    ldu<DT>(p, (i64)col, v);
+  } else if constexpr (K == 'b' || K == 'c') {
+    const float x = ld1<DT>(p, K == 'b' ? 0 : (i64)row);
+    for (int j = 0; j < EW_V; ++j) v[j] = x;
+  } else {
+    for (int j = 0; j < EW_V; ++j) {
+      const u32 t = col + j;
+      const bool per_col = K == 'w' || K == 'W', one = K == 'w' || K == 'd';
+      const u32 past = one ? (t >= d3 ? 1u : 0u) : t / d3;
+      v[j] = ld1<DT>(p, (i64)(per_col ? t - past * d3 : row + past));
+    }
   }
 }
 // EW_V (4 or 8) elements per lane, defined by the generated source.  The access form K of
@@ -449,10 +535,11 @@ static std::string ew_logistic_t(const ihip_ew_instr* code, int pe, int u_reg,
 // the staged inputs) and the other inputs from the registers they were prefetched into.
 // preload (untiled form only): every LOAD was issued ahead into L<pc>[u] (u: the lane's row of
 // the trip; L<pc>[0] for the row-invariant inputs of `rowinv`) and becomes a register copy;
-// stores are predicated on live[u] and address row rb + u.
+// stores are predicated on live[u] and address row rb + u.  flat: preloaded the same way, stores
+// go to element e[u].
 static std::string ew_jit_body(const ihip_ew_instr* code, int n_code, const int* in_dt, const int* out_dt,
                                const char* in_kind, const char* out_kind, bool tiled, const char* ind,
-                               bool preload = false, uint32_t rowinv = 0) {
+                               bool preload = false, uint32_t rowinv = 0, bool flat = false) {
   std::string s;
   std::vector<int> fuse_u(n_code), fuse_e(n_code);
   std::vector<char> skip_v(n_code);
@@ -510,7 +597,9 @@ static std::string ew_jit_body(const ihip_ew_instr* code, int n_code, const int*
                    in.a == 0 ? "c0" : in.a == 1 ? "c1" : in.a == 2 ? "c2" : "c3 + j");
         break;
       case IHIP_EW_STORE:
-        if (preload)
+        if (flat)
+          s += fmt("%sif (live[u]) stu<%d>(a.out_ptr[%d], (i64)e[u], r[%d]);\n", ind, out_dt[in.b], in.b, in.a);
+        else if (preload)
           s += fmt("%sif (live[u]) stk<%d, '%c'>(a.out_ptr[%d], (rb + u) * D3 + c3, valid, r[%d]);\n", ind,
                    out_dt[in.b], out_kind[in.b], in.b, in.a);
         else
@@ -717,6 +806,59 @@ std::string ew_jit_source(const ihip_ew_instr* code, int n_code, int n_inputs, c
   return s;
 }
 
+// Flat form (plan_flat): every lane takes EW_V consecutive elements of the whole iteration space,
+// EW_U such runs per trip with their loads issued together.  The last run starts EW_V before the
+// end and repeats elements of the one before it (the same values are stored twice), so no run is
+// partial and no load sits behind a branch.
+std::string ew_jit_source_flat(const ihip_ew_instr* code, int n_code, int n_inputs, const int* in_dt, int n_outputs,
+                               const int* out_dt, const char* in_kind) {
+  const int V = ew_jit_width(n_inputs, in_dt, n_outputs, out_dt);
+  int nreg = IHIP_EW_MAX_REGS;
+  for (int pc = 0; pc < n_code; ++pc)
+    if (code[pc].op != IHIP_EW_STORE && code[pc].dst + 1 > nreg) nreg = code[pc].dst + 1;
+  uint32_t scalars = 0;
+  bool rows = false;
+  for (int k = 0; k < n_inputs; ++k) {
+    if (in_kind[k] == 'b') scalars |= 1u << k;
+    rows |= in_kind[k] != 'b' && in_kind[k] != 'u';
+  }
+  std::string s = fmt("#define EW_V %d\n#define EW_NREG %d\n#define EW_U %d\n", V, nreg,
+                      ew_jit_rows_per_trip(code, n_code, V, scalars));
+  s += kPrelude;
+  s += "extern \"C\" __global__ __launch_bounds__(256) void ihip_ew_jit(const EwJitArgs a) {\n"
+       "  const u32 d3 = (u32)a.shape[3], nrun = (a.total + EW_V - 1) / EW_V;\n";
+  for (int pc = 0; pc < n_code; ++pc)
+    if (code[pc].op == IHIP_EW_LOAD && ((scalars >> code[pc].a) & 1u))
+      s += fmt("  float L%d[1][EW_V];\n  ldf<%d, 'b'>(a.in_ptr[%d], 0, 0, 0, d3, L%d[0]);\n", pc, in_dt[code[pc].a],
+               (int)code[pc].a, pc);
+  s += "  for (u32 t0 = blockIdx.x * (256 * EW_U); t0 < nrun; t0 += gridDim.x * (256 * EW_U)) {\n"
+       "    u32 e[EW_U], row[EW_U], col[EW_U];\n"
+       "    bool live[EW_U];\n"
+       "#pragma unroll\n"
+       "    for (int u = 0; u < EW_U; ++u) {\n"
+       "      const u32 run = t0 + u * 256 + threadIdx.x;\n"
+       "      live[u] = run < nrun;\n"
+       "      e[u] = run < nrun - 1 ? run * EW_V : a.total - EW_V;\n";
+  s += rows ? "      row[u] = (u32)(((unsigned long long)e[u] * a.magic) >> a.shift);\n"
+              "      col[u] = e[u] - row[u] * d3;\n"
+            : "      row[u] = 0;\n      col[u] = 0;\n";
+  s += "    }\n";
+  for (int pc = 0; pc < n_code; ++pc) {
+    if (code[pc].op != IHIP_EW_LOAD || ((scalars >> code[pc].a) & 1u)) continue;
+    const int k = code[pc].a;
+    s += fmt("    float L%d[EW_U][EW_V];\n"
+             "#pragma unroll\n"
+             "    for (int u = 0; u < EW_U; ++u) ldf<%d, '%c'>(a.in_ptr[%d], e[u], row[u], col[u], d3, L%d[u]);\n",
+             pc, in_dt[k], in_kind[k], k, pc);
+  }
+  s += "#pragma unroll\n"
+       "    for (int u = 0; u < EW_U; ++u) {\n"
+       "      float r[EW_NREG][EW_V];\n";
+  s += ew_jit_body(code, n_code, in_dt, out_dt, in_kind, in_kind, false, "      ", true, scalars, true);
+  s += "    }\n  }\n}\n";
+  return s;
+}
+
 namespace {
 
 // One specialised program: its code object, and the module loaded from it on each device.
@@ -774,6 +916,59 @@ struct JitPlan {
   std::string src;
   unsigned gx = 0, gy = 0;
 };
+
+// Rewrites the plan to the flat form where it applies and is the better one.  It applies when
+// every output and input is one value per element of the iteration space in memory order, per
+// column, per row or one for all (no iota: a run has no single row), and the space has at least
+// one run and less than 2^31 elements.  It is taken when the row form would leave an operand
+// without full vectors (D3 % V != 0, or a base off its vector's alignment: `vectors` false), 30%
+// of the lanes of the waves that a row occupies idle, or, for rows of several workgroups, a quarter
+// of their lanes.  Measured in us, row form -> flat form: without vectors, bf16 sigmoid [4096, 12289]
+// 126.6 -> 38.0 (5.3 TB/s), [1000000, 23] 627.8 -> 19.9, f32 bias + ReLU [8192, 4099] 83.4 -> 52.0,
+// [65536, 257] 49.2 -> 27.5, [262144, 24] 37.9 -> 11.2; idle lanes, f32 [400000, 64] 59.6 -> 35.2,
+// [150000, 168] (66% of a wave) 37.1 -> 36.3, [60000, 1040] (51% of two workgroups) 108.3 -> 84.3,
+// bf16 [100000, 200] 28.2 -> 18.0, [40000, 1040] 37.2 -> 33.0, [8192, 2600] 22.3 -> 19.2; on the
+// other side f32 [100000, 200] (78%) 29.7 -> 30.2, [60000, 512] 41.4 -> 43.5, [8192, 8192] 85.2 -> 89.0,
+// bf16 [20000, 4096] 58.6 -> 60.2.
+bool plan_flat(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inputs, int n_inputs, const int* in_dt,
+               int n_outputs, const int* out_dt, const int64_t (&shape)[4], bool vectors, int V, JitPlan& pl) {
+  EwJitArgs& a = pl.a;
+  const int64_t D3 = shape[3], total = a.rows * D3;
+  const int64_t wave_lanes = (a.nvec + 63) / 64 * 64, wg_lanes = (a.nvec + 255) / 256 * 256;
+  const bool idle = a.nvec * 10 < wave_lanes * 7 || (a.nvec > 256 && a.nvec * 4 < wg_lanes * 3);
+  if (total < V || total >= (int64_t(1) << 31) - 256 * 4 * 8 || (vectors && !idle)) return false;
+  for (int pc = 0; pc < n_code; ++pc)
+    if (code[pc].op == IHIP_EW_IOTA) return false;
+  char kind[IHIP_EW_NATIVE_MAX_INPUTS + 1] = {};
+  const char per_col = D3 % V == 0 ? 'x' : D3 >= V ? 'w' : 'W', per_row = D3 % V == 0 ? 'c' : D3 >= V ? 'd' : 'D';
+  for (int k = 0; k < n_inputs; ++k) {
+    const int64_t* st = inputs[k].stride;
+    // the operand's stride along axis d is `want` (or the axis has one element)
+    const auto is = [&](int d, int64_t want) { return shape[d] == 1 || st[d] == want; };
+    const int64_t r2 = shape[2], r1 = shape[1] * shape[2];
+    if (is(3, 1) && is(2, D3) && is(1, r2 * D3) && is(0, r1 * D3)) kind[k] = 'u';
+    else if (is(3, 0) && is(2, 0) && is(1, 0) && is(0, 0)) kind[k] = 'b';
+    else if (is(3, 1) && is(2, 0) && is(1, 0) && is(0, 0)) kind[k] = per_col;
+    else if (is(3, 0) && is(2, 1) && is(1, r2) && is(0, r1)) kind[k] = per_row;
+    else return false;
+  }
+  a.total = static_cast<uint32_t>(total);
+  // floor(e / D3) for e < 2^31: with l = ceil(log2 D3), magic = floor(2^(31+l) / D3) + 1 exceeds
+  // 2^(31+l) / D3 by at most 1, so (e * magic) / 2^(31+l) exceeds e / D3 by at most e / 2^(31+l) <
+  // 2^-l <= 1 / D3: it never reaches the next integer.  magic < 2^32 because D3 > 2^(l-1).
+  int l = 0;
+  while ((int64_t(1) << l) < D3) ++l;
+  a.shift = static_cast<uint32_t>(31 + l);
+  a.magic = static_cast<uint32_t>(((static_cast<unsigned __int128>(1) << (31 + l)) / D3) + 1);
+  pl.src = ew_jit_source_flat(code, n_code, n_inputs, in_dt, n_outputs, out_dt, kind);
+  uint32_t scalars = 0;
+  for (int k = 0; k < n_inputs; ++k) scalars |= kind[k] == 'b' ? 1u << k : 0u;
+  const int64_t per_wg = 256 * V * static_cast<int64_t>(ew_jit_rows_per_trip(code, n_code, V, scalars));
+  const int64_t wgs = (total + per_wg - 1) / per_wg;
+  pl.gx = static_cast<unsigned>(wgs < 65536 ? wgs : 65536);
+  pl.gy = 1;
+  return true;
+}
 
 // Plans a launch: the access form of every operand (see ldk), the LDS-staged inputs, the
 // arguments and the grid.  Returns false for an empty iteration space (nothing to launch).
@@ -834,6 +1029,13 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     const int64_t* st = inputs[k].stride;
     if ((st[0] == 0 || shape[0] == 1) && (st[1] == 0 || shape[1] == 1) && (st[2] == 0 || shape[2] == 1))
       rowinv |= 1u << k;
+  }
+  if (tile_mask == 0) {
+    const char full = V == 8 ? '8' : '4';
+    bool vectors = true;
+    for (int k = 0; k < n_inputs; ++k) vectors &= in_kind[k] == full || in_kind[k] == 'b';
+    for (int k = 0; k < n_outputs; ++k) vectors &= out_kind[k] == full;
+    if (plan_flat(code, n_code, inputs, n_inputs, in_dt, n_outputs, out_dt, shape, vectors, V, pl)) return true;
   }
   pl.src = ew_jit_source(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind, out_kind, rowinv);
   if (tile_mask != 0) {  // one workgroup per 64 x 64 tile (linear id; grid-strided beyond the grid limits)

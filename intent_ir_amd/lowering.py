@@ -34,7 +34,7 @@ from typing import Any, Dict, List, Mapping, Optional, Tuple
 from .ir import IntentFunction, ScheduleSketch, as_intent, resolve_shape
 from .macros import GELU_CUBIC, GELU_NEG_2_SQRT_2_OVER_PI, expand_macros
 from .opset import HIP_SUPPORTED_OPS
-from .ewprogram import BINARY as EW_BINARY, DTYPE_CODE as EW_DTYPE_CODE, UNARY as EW_UNARY
+from .ewprogram import BINARY as EW_BINARY, DTYPE_CODE as EW_DTYPE_CODE, OP as EW_OP, UNARY as EW_UNARY
 from .ewprogram import EwCompileError, EwLimitError, compile_elementwise
 from .patterns import ExprBuilder, PatternError, close, unify
 
@@ -972,7 +972,8 @@ def _ew_launch(prog, dtype_of) -> HipLaunch:
     outputs: lanes own 8 elements when every operand is 16-bit or narrower, else 4.  Inputs read
     across their unit-stride axis (axis 2 contiguous, axis 3 strided; up to 4) select the
     LDS-tiled form: one workgroup per 64 x 64 tile, a 64 x 65 f32 tile each.  Otherwise up to
-    16384 256-lane workgroups stride over groups of U rows and over vectors."""
+    16384 256-lane workgroups stride over groups of U rows and over vectors, or (_ew_flat_workgroups)
+    over the whole space as one run of elements."""
     sh = [1] * (4 - len(prog.shape)) + [int(d) for d in prog.shape]
     narrow = all(dtype_of(n) in ("f16", "bf16", "bool", "i1", "u8") for n in [i for i, _ in prog.inputs] + list(prog.outputs))
     v = 8 if narrow else 4
@@ -985,6 +986,9 @@ def _ew_launch(prog, dtype_of) -> HipLaunch:
         tx, ty = _cdiv(sh[3], 64), sh[0] * sh[1] * _cdiv(sh[2], 64)
         return HipLaunch((max(1, min(tx, 65535)), max(1, min(ty, 65535)), 1), (256, 1, 1), tiled * 64 * 65 * 4)
     rows = sh[0] * sh[1] * sh[2]
+    flat = _ew_flat_workgroups(prog, sh, v)
+    if flat:
+        return HipLaunch((flat, 1, 1), (256, 1, 1), 0)
     gx = max(1, min(1024, _cdiv(_cdiv(sh[3], v), 256)))
     # a lane takes U rows per trip, U = 64 // (row-varying loads x elements per lane) in 1..4
     # (ew_jit_rows_per_trip); inputs with zero stride or extent 1 on axes 0-2 do not count
@@ -992,6 +996,37 @@ def _ew_launch(prog, dtype_of) -> HipLaunch:
     loads = sum(1 for ins in prog.code if ins[0] == 1 and not rowinv[ins[2]])
     U = 4 if loads == 0 else max(1, min(4, 64 // (loads * v)))
     return HipLaunch((gx, max(1, min(_cdiv(rows, U), 65535, _cdiv(16384, gx))), 1), (256, 1, 1), 0)
+
+
+def _ew_flat_workgroups(prog, sh, v: int) -> int:
+    """Workgroups of the flat form (ewjit.hip plan_flat), 0 where it is not taken: operands that are
+    one value per element in memory order, per column, per row or one for all, no iota, and rows that
+    would leave an operand without full vectors, 30% of the lanes of its waves idle, or a quarter of
+    the lanes of several workgroups."""
+    d0, d1, d2, d3 = sh
+    rows = d0 * d1 * d2
+    total, nvec = rows * d3, _cdiv(d3, v)
+    iota = any(ins[0] == EW_OP["iota"] for ins in prog.code)
+    if iota or not v <= total < (1 << 31) - 8192:
+        return 0
+
+    def full(st):  # whole V-element vectors in the row form, or one value along the row
+        return st[3] == 0 or (d3 % v == 0 and st[3] == 1 and all(st[d] % v == 0 or sh[d] == 1 for d in range(3)))
+
+    vectors = d3 % v == 0 and all(full(st) for _, st in prog.inputs)
+    idle = nvec * 10 < _cdiv(nvec, 64) * 64 * 7 or (nvec > 256 and nvec * 4 < _cdiv(nvec, 256) * 256 * 3)
+    if vectors and not idle:
+        return 0
+    forms = ((d1 * d2 * d3, d2 * d3, d3, 1), (0, 0, 0, 0), (0, 0, 0, 1), (d1 * d2, d2, 1, 0))
+    one = []  # inputs that are one value for all: not loaded per run
+    for _, st in prog.inputs:
+        f = next((i for i, want in enumerate(forms) if all(sh[d] == 1 or st[d] == want[d] for d in range(4))), None)
+        if f is None:
+            return 0
+        one.append(f == 1)
+    loads = sum(1 for ins in prog.code if ins[0] == 1 and not one[ins[2]])
+    u = 4 if loads == 0 else max(1, min(4, 64 // (loads * v)))
+    return min(65536, _cdiv(total, 256 * v * u))
 
 
 def call_args_to_json(call_args) -> List[Dict[str, Any]]:
