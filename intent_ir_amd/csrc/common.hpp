@@ -21,6 +21,10 @@ constexpr int kNumXcd = 8;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// The same at any 2-byte boundary (rows of an odd number of 16-bit elements): gfx950 takes a
+// vector access at any address, so such a row still moves 16 bytes per lane.
+typedef uint32_t u32x4_b2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_b2 __attribute__((ext_vector_type(2), aligned(2)));
 
 // ---------------------------------------------------------------- 16-bit floats
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {

@@ -2,7 +2,7 @@
 // f32 accumulation on v_mfma_f32_32x32x16_bf16, C bf16 (RNE).  Any M, N and K as long as
 // every row of A and B starts 16-byte aligned (K % 8 == 0, M % 8 == 0 when A is given as
 // [K,M], N % 8 == 0 when B is given as [K,N]) and the bases are 16-byte aligned; C rows that
-// are not (N % 8 != 0 with B given as [N,K]) are written with 2-byte stores.  Other shapes
+// are not (N % 8 != 0 with B given as [N,K]) are written with 16-byte stores at any 2-byte boundary.  Other shapes
 // take the guarded kernel in gemm.hip.  Edge tiles (past M or N, or all tiles when K is not a
 // multiple of DK) copy through range-checked buffer descriptors: reads past the end of a
 // tensor and k-chunks past K load zeros, and what an edge tile reads outside [M) x [N) only
@@ -493,7 +493,7 @@ constexpr int fast_lds_bytes() {
 }
 
 // One TILE x TILE C tile at (m0, n0); lds_raw is the kernel's LDS.  CU: C rows are not 16-byte
-// aligned (N % 8 != 0, only with B given as [N, K]); C is then written with 2-byte stores.
+// aligned (N % 8 != 0, only with B given as [N, K]); C is then stored at 2-byte boundaries.
 // kPartial (split-K): the tile's f32 sums over R's K segment go to P (row-major, ldp floats
 // per row) instead of bias + activation into C.
 template <int DK, int STAGES, bool AKM, bool BKM, bool EDGE, int TILE, bool CU, bool kPartial = false>
@@ -772,9 +772,13 @@ __device__ __forceinline__ void gemm_fast_tile(const uint16_t* __restrict__ A, c
     if constexpr (CU) {
       if (!EDGE || (col_ok && m0 + row < M)) {
         uint16_t* dst = C + (m0 + row) * N + n0 + chunk * 8;
+        if (!EDGE || col_left >= 8) {
+          *reinterpret_cast<u32x4_b2*>(dst) = v;
+        } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (!EDGE || e < col_left) dst[e] = static_cast<uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+          for (int e = 0; e < 7; ++e)
+            if (e < col_left) dst[e] = static_cast<uint16_t>(v[e >> 1] >> (16 * (e & 1)));
+        }
       }
     } else {
       if (!EDGE || (col_ok && m0 + row < M)) *reinterpret_cast<u32x4*>(C + (m0 + row) * N + n0 + chunk * 8) = v;
@@ -846,8 +850,8 @@ void gemm_bf16_splitk_kernel(const uint16_t* __restrict__ A, const uint16_t* __r
 }
 
 // C = act(sum over the S segments of P + bias) in bf16 (round to nearest even), segments added
-// in order 0 .. S-1; one thread per 4 consecutive columns of a row.  C rows are written with
-// one 8-byte store where 8-byte aligned, else with 2-byte stores.
+// in order 0 .. S-1; one thread per 4 consecutive columns of a row, one 8-byte store each at any
+// 2-byte boundary.
 __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float* __restrict__ P, int S, int64_t M, int64_t N,
                                                           int64_t ldp, const float* __restrict__ bias, int relu,
                                                           uint16_t* __restrict__ C) {
@@ -877,11 +881,11 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(const float* __restric
     v[q] = __builtin_elementwise_maximum(sum[q] + (bias != nullptr && n + q < N ? bias[n + q] : 0.0f), floor_v);
   uint16_t* dst = C + m * N + n;
   const u32x2 pk = {pack_bf16x2_rne(v[0], v[1]), pack_bf16x2_rne(v[2], v[3])};
-  if (n + 4 <= N && (reinterpret_cast<uintptr_t>(dst) & 7) == 0) {
-    *reinterpret_cast<u32x2*>(dst) = pk;
+  if (n + 4 <= N) {
+    *reinterpret_cast<u32x2_b2*>(dst) = pk;
   } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 3; ++q)
       if (n + q < N) dst[q] = static_cast<uint16_t>(pk[q >> 1] >> (16 * (q & 1)));
   }
 }
@@ -903,7 +907,7 @@ constexpr int64_t kSkinnyRows = 128;
 // masks) as long as every row of A and B starts 16 bytes aligned: K % 8 == 0, M % 8 == 0 when
 // A is given as [K, M], and N % 8 == 0 when B is given as [K, N].  With B given as [N, K]
 // (the layout of a linear layer's weight) N may be anything: C rows that are not 16-byte
-// aligned are written with 2-byte stores.  When K is not a whole number of K steps, A and B
+// aligned are stored 16 bytes at a time all the same.  When K is not a whole number of K steps, A and B
 // must be below 2 GiB each (the ragged k-chunks are pointed past every record).
 bool gemm_fast_fits(int64_t M, int64_t N, int64_t K, bool transpose_a, bool transpose_b, const void* A, const void* B,
                     const void* C) {
@@ -956,7 +960,7 @@ static void launch_tiles(const uint16_t* A, const uint16_t* B, const float* bias
 
 // transpose_a: A is given as [K, M]; transpose_b: B is given as [N, K].  tile: 0 = by grid
 // size (gemm_fast_tile_extent), else 128 or 256.  c_unaligned: C's base is not 16-byte aligned
-// (only with transpose_b): C is written with 2-byte stores, as for N % 8 != 0.
+// (only with transpose_b): C is stored as for N % 8 != 0.
 hipError_t launch_gemm_fast(const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, int64_t M, int64_t N,
                             int64_t K, bool transpose_a, bool transpose_b, int relu, int tile, hipStream_t s,
                             bool c_unaligned) {

@@ -3,14 +3,13 @@
 // [K, M], or 2-byte aligned bases) are first copied into a caller workspace as K-contiguous
 // rows of K8 = K rounded up to 8 elements, zero past K, and the tiled kernel then runs on the
 // copies (A as [M, K8], B as [N, K8]; C rows that are not 16-byte aligned are written with
-// 2-byte stores).  The zeros past K add exact zeros in the k slots the guarded kernel also
+// 16-byte stores at their own 2-byte boundaries).  The zeros past K add exact zeros in the k slots the guarded kernel also
 // fills with zeros, and both kernels issue the same MFMAs in the same k order, so the result
 // is bit-identical to the guarded kernel's.
 //
 // Packing is one HBM pass per packed operand (read R x K, write R x K8 elements):
-//  * a K-contiguous source (A [M, K], B [N, K]) is re-pitched row by row: each thread writes
-//    8 consecutive elements (one 16-byte store) from 4-byte loads when every row starts
-//    4-byte aligned (K even), else from 2-byte loads;
+//  * a K-contiguous source (A [M, K], B [N, K]) is re-pitched row by row: each thread moves 8
+//    consecutive elements, read at the source row's own 2-byte boundary;
 //  * a K-major source (A [K, M], B [K, N]) is transposed through LDS in 64 x 64 tiles, read
 //    along source rows and written in 16-byte stores along destination rows.
 //
@@ -125,60 +124,54 @@ hipError_t launch_tiled(const uint16_t* A, const uint16_t* B, const float* bias,
 bool shape_packs_a(int64_t M, int64_t K, bool ta) { return K % 8 != 0 || (ta && M % 8 != 0); }
 bool shape_packs_b(int64_t N, int64_t K, bool tb) { return K % 8 != 0 || (!tb && N % 8 != 0); }
 
-// dst [R, K8] from a K-contiguous src [R, K] (leading dimension K); kPairs: every row starts
-// 4-byte aligned (K even, src 4-byte aligned), so pairs of elements load as one dword.
-template <bool kPairs>
+// dst [R, K8] from a K-contiguous src [R, K] (leading dimension K): 16 bytes per thread, read at
+// the row's own 2-byte boundary.
 __global__ __launch_bounds__(256) void pack_rows_kc(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                     int64_t R, int64_t K, int64_t K8) {
   const int64_t chunks = K8 / 8;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= R * chunks) return;
   const int64_t r = t / chunks, k0 = (t % chunks) * 8;
-  const uint16_t* s = src + r * K;
-  uint32_t w[4];
+  const uint16_t* s = src + r * K + k0;
+  u32x4 w = {0, 0, 0, 0};
+  if (k0 + 8 <= K) {
+    w = *reinterpret_cast<const u32x4_b2*>(s);
+  } else {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int64_t k = k0 + 2 * e;
-    if (kPairs) {  // K even: a pair is wholly inside the row or wholly past it
-      w[e] = k < K ? *reinterpret_cast<const uint32_t*>(s + k) : 0u;
-    } else {
-      const uint32_t lo = k < K ? s[k] : 0u, hi = k + 1 < K ? s[k + 1] : 0u;
-      w[e] = lo | (hi << 16);
-    }
+    for (int e = 0; e < 7; ++e)
+      if (k0 + e < K) w[e >> 1] |= static_cast<uint32_t>(s[e]) << (16 * (e & 1));
   }
-  *reinterpret_cast<u32x4*>(dst + r * K8 + k0) = u32x4{w[0], w[1], w[2], w[3]};
+  *reinterpret_cast<u32x4*>(dst + r * K8 + k0) = w;
 }
 
 // dst [R, K8] from a K-major src [K, R] (leading dimension R): 64 x 64 tiles through LDS.
-// Reads go along src rows (4-byte loads when every row starts 4-byte aligned, kPairs), writes
-// along dst rows in 16-byte stores, 8 lanes per 128-byte row piece.
+// Reads go along src rows, 16 bytes per lane at the row's own 2-byte boundary, writes along dst
+// rows in 16-byte stores, 8 lanes per 128-byte row piece.
 constexpr int kT = 64;
-template <bool kPairs>
 __global__ __launch_bounds__(256) void pack_rows_km(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                     int64_t R, int64_t K, int64_t K8) {
-  __shared__ uint16_t tile[kT][kT + 2];
+  __shared__ __attribute__((aligned(4))) uint16_t tile[kT][kT + 2];
   const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kT, k0 = static_cast<int64_t>(blockIdx.y) * kT;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // read: src row k0 + i holds r0 .. r0+63 contiguously
-  if constexpr (kPairs) {
-    const int c = 2 * (lane & 31);
-    for (int i = 2 * w + (lane >> 5); i < kT; i += 8) {
-      const int64_t k = k0 + i, r = r0 + c;
-      uint32_t v = 0;
-      if (k < K && r + 1 < R) {
-        v = *reinterpret_cast<const uint32_t*>(src + k * R + r);
-      } else if (k < K && r < R) {
-        v = src[k * R + r];
-      }
-      tile[i][c] = static_cast<uint16_t>(v);
-      tile[i][c + 1] = static_cast<uint16_t>(v >> 16);
-    }
-  } else {
-    for (int i = w; i < kT; i += 4) {
-      const int64_t k = k0 + i, r = r0 + lane;
-      tile[i][lane] = (k < K && r < R) ? src[k * R + r] : 0;
+  const int c = 8 * (threadIdx.x & 7);
+  u32x4 v[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int64_t k = k0 + 32 * p + (threadIdx.x >> 3), r = r0 + c;
+    v[p] = u32x4{0, 0, 0, 0};
+    if (k < K && r + 8 <= R) {
+      v[p] = *reinterpret_cast<const u32x4_b2*>(src + k * R + r);
+    } else if (k < K) {
+#pragma unroll
+      for (int e = 0; e < 7; ++e)
+        if (r + e < R) v[p][e >> 1] |= static_cast<uint32_t>(src[k * R + r + e]) << (16 * (e & 1));
     }
   }
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(&tile[32 * p + (threadIdx.x >> 3)][c + 2 * e]) = v[p][e];
   __syncthreads();
   // write: dst row r0 + i gets k0 .. k0+63 (zeros past K; K8, a multiple of 8, may end inside
   // the tile), 8 columns per lane
@@ -200,16 +193,10 @@ hipError_t pack(const uint16_t* src, uint16_t* dst, int64_t R, int64_t K, bool k
   if (!kmajor) {
     const int64_t threads = R * (K8 / 8);
     const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
-    if (K % 2 == 0 && (reinterpret_cast<uintptr_t>(src) & 3) == 0)
-      pack_rows_kc<true><<<grid, dim3(256), 0, s>>>(src, dst, R, K, K8);
-    else
-      pack_rows_kc<false><<<grid, dim3(256), 0, s>>>(src, dst, R, K, K8);
+    pack_rows_kc<<<grid, dim3(256), 0, s>>>(src, dst, R, K, K8);
   } else {
     const dim3 grid(static_cast<unsigned>((R + kT - 1) / kT), static_cast<unsigned>((K8 + kT - 1) / kT));
-    if (R % 2 == 0 && (reinterpret_cast<uintptr_t>(src) & 3) == 0)
-      pack_rows_km<true><<<grid, dim3(256), 0, s>>>(src, dst, R, K, K8);
-    else
-      pack_rows_km<false><<<grid, dim3(256), 0, s>>>(src, dst, R, K, K8);
+    pack_rows_km<<<grid, dim3(256), 0, s>>>(src, dst, R, K, K8);
   }
   return hipGetLastError();
 }
@@ -259,7 +246,7 @@ hipError_t launch_gemm_packed(const uint16_t* A, const uint16_t* B, const float*
   const int64_t K8 = round8(K);
   const bool c_unaligned = N % 8 != 0 || (reinterpret_cast<uintptr_t>(C) & 15) != 0;
   const bool pa = shape_packs_a(M, K, ta) || (reinterpret_cast<uintptr_t>(A) & 15) != 0;
-  // C written with 2-byte stores needs B as [N, K]: pack B then too
+  // C stored at 2-byte boundaries needs B as [N, K]: pack B then too
   const bool pb = shape_packs_b(N, K, tb) || (reinterpret_cast<uintptr_t>(B) & 15) != 0 || (c_unaligned && !tb);
   const int64_t a_bytes = pa ? align_up(M * K8 * 2) : 0, b_bytes = pb ? align_up(N * K8 * 2) : 0;
   if (a_bytes + b_bytes > ws_bytes) return hipErrorNotSupported;
@@ -272,7 +259,7 @@ hipError_t launch_gemm_packed(const uint16_t* A, const uint16_t* B, const float*
   const uint16_t* B2 = pb ? b_ws : B;
   const bool ta2 = pa ? false : ta, tb2 = pb ? true : tb;
   // the tiled kernel's conditions on the packed operands (C's alignment is handled by the
-  // 2-byte store path; a 16-byte aligned stand-in is passed for it)
+  // unaligned store path; a 16-byte aligned stand-in is passed for it)
   if (!gemm_fast_fits(M, N, K8, ta2, tb2, A2, B2, ws)) return hipErrorNotSupported;
   hipError_t e = hipSuccess;
   if (pa) e = pack(A, a_ws, M, K, ta, s);
