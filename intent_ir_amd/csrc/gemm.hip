@@ -4,8 +4,9 @@
 //
 // Entry point of the GEMM family: shapes whose rows all start 16-byte aligned (N % 8 == 0,
 // K % 8 == 0, M % 8 == 0 for a transposed A) with 16-byte aligned operands go to
-// gemm_fast.hip, for any M, N and K; every other shape runs the guarded kernel below, which
-// stages operands through registers:
+// gemm_fast.hip, for any M, N and K; products with one small side to gemm_direct.hip (with the
+// automatic tile); every other shape runs the guarded kernel below, which stages operands through
+// registers:
 //  * workgroup tile TB(M) x TB(N), TB = 256, or 128 for grids of at most 128 tiles of 256x256
 //    (half the CUs; as in gemm_fast.hip), K step 64; 256 threads = 4 waves in a 2x2 grid,
 //    each wave owning a TB/2 x TB/2 sub-tile = (TB/64)^2 blocks of v_mfma_f32_32x32x16_bf16;
@@ -266,6 +267,10 @@ static hipError_t launch_guarded_tb(const uint16_t* A, const uint16_t* B, const 
 }
 
 int gemm_fast_tile_extent(int64_t M, int64_t N);
+bool gemm_direct_takes(int64_t M, int64_t N, int64_t K, bool transpose_a, bool transpose_b);
+hipError_t launch_gemm_direct(const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, int64_t M,
+                              int64_t N, int64_t K, bool transpose_b, int relu, void* ws, int64_t ws_bytes,
+                              hipStream_t s);
 
 // tile: 0 = automatic (256x256 tiles, 128x128 for grids of at most 128 256x256 tiles), else
 // 128 or 256; the same rule and choice for the tiled and the guarded kernel.
@@ -273,6 +278,8 @@ hipError_t launch_gemm_bf16_bias_relu(const uint16_t* A, const uint16_t* B, cons
                                       int64_t N, int64_t K, bool transpose_a, bool transpose_b, int relu, int tile,
                                       hipStream_t s) {
   if (M == 0 || N == 0) return hipSuccess;
+  if (tile == 0 && gemm_direct_takes(M, N, K, transpose_a, transpose_b))
+    return launch_gemm_direct(A, B, bias, C, M, N, K, transpose_b, relu, nullptr, 0, s);
   if (gemm_fast_fits(M, N, K, transpose_a, transpose_b, A, B, C))
     return launch_gemm_fast(A, B, bias, C, M, N, K, transpose_a, transpose_b, relu, tile, s, false);
   const int tb = tile != 0 ? tile : gemm_fast_tile_extent(M, N);
@@ -288,6 +295,8 @@ hipError_t launch_gemm_bf16_bias_relu_ws(const uint16_t* A, const uint16_t* B, c
                                          int64_t M, int64_t N, int64_t K, bool transpose_a, bool transpose_b, int relu,
                                          int tile, void* ws, int64_t ws_bytes, hipStream_t s) {
   if (M == 0 || N == 0) return hipSuccess;
+  if (tile == 0 && gemm_direct_takes(M, N, K, transpose_a, transpose_b))
+    return launch_gemm_direct(A, B, bias, C, M, N, K, transpose_b, relu, ws, ws_bytes, s);
   // split-K by the split rule when the workspace holds the partials, else unsplit
   hipError_t e = launch_gemm_split(A, B, bias, C, M, N, K, transpose_a, transpose_b, relu, tile, 0, ws, ws_bytes, s);
   if (e != hipErrorNotSupported) return e;

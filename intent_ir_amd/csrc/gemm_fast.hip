@@ -980,6 +980,9 @@ hipError_t launch_gemm_fast(const uint16_t* A, const uint16_t* B, const float* b
   return hipGetLastError();
 }
 
+hipError_t launch_splitk_reduce(const float* P, int S, int64_t M, int64_t N, int64_t ldp, const float* bias, int relu,
+                                uint16_t* C, hipStream_t s);
+
 // Split-K with S segments of kseg k (gemm_split_k): the tiled kernel writes f32 partials to P
 // (S x M x ldp floats) and gemm_splitk_reduce adds them in order with bias and activation.
 // Same operand conditions as launch_gemm_fast; C may have any alignment.
@@ -1008,7 +1011,12 @@ hipError_t launch_gemm_splitk(const uint16_t* A, const uint16_t* B, const float*
   else
     launch_splitk_tiles<128>(A, B, P, M, N, K, kseg, S, ldp, transpose_a, transpose_b, s);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  return e != hipSuccess ? e : launch_splitk_reduce(P, S, M, N, ldp, bias, relu, C, s);
+}
+
+// C from the S planes of partial sums at P (M x ldp floats each).
+hipError_t launch_splitk_reduce(const float* P, int S, int64_t M, int64_t N, int64_t ldp, const float* bias, int relu,
+                                uint16_t* C, hipStream_t s) {
   const int64_t threads = M * (ldp / 4);
   gemm_splitk_reduce<<<dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s>>>(P, S, M, N, ldp, bias,
                                                                                              relu, C);

@@ -313,6 +313,7 @@ def _match_gemm(c: _Ctx) -> Optional[HipLoweredKernel]:
     # (rows that cannot start 16-byte aligned), or the guarded kernel, as gemm_fast_fits and
     # launch_gemm_packed decide for 16-byte aligned tensors; the tiled path split along K into
     # S segments when the grid has too few tiles (gemm_pack.hip split_plan)
+    direct = tile == 0 and gemm_direct_takes(M, N, K, ta, tb)
     full = _gemm_fast_fits(M, N, K, ta, tb)
     pack_ws = 0 if full else gemm_pack_bytes(M, N, K, ta, tb)
     K8 = _cdiv(K, 8) * 8
@@ -335,6 +336,9 @@ def _match_gemm(c: _Ctx) -> Optional[HipLoweredKernel]:
         launch = HipLaunch(grid, (256, 1, 1), _gemm_fast_lds(t, ta2 if packed else ta))
     else:  # guarded kernel: the same tile choice, a double-buffered {A, Bt} tile pair of 64-k slices
         launch = HipLaunch(grid, (256, 1, 1), 147456 if t == 256 else 73728)
+    if direct:  # one small side: gemm_direct.hip, with or without segments of K in the workspace
+        launch, S = _gemm_direct_launch(M, N, K, tb)
+        ws = _gemm_split_bytes(M, N, S)
     if ws > 0:
         args = [("tensor", a), ("tensor", b), ("tensor", env["bias"][1]) if has_bias else ("null", None),
                 ("tensor", oname), ("i64", M), ("i64", N), ("i64", K), ("i32", int(ta)), ("i32", int(tb)),
@@ -344,6 +348,43 @@ def _match_gemm(c: _Ctx) -> Optional[HipLoweredKernel]:
     kid = ("ihip_gemm_bf16_bias_relu_ex" if tile else "ihip_gemm_bf16_bias_relu_t" if (ta or tb)
            else "ihip_gemm_bf16_bias_relu")
     return HipLoweredKernel(c.fn.name, kid, c.io(names), launch, [oname], dict(c.b), tuple(args))
+
+
+def gemm_direct_takes(M: int, N: int, K: int, ta: bool, tb: bool) -> bool:
+    """gemm_direct.hip gemm_direct_takes."""
+    if ta or M < 1 or not 16 <= N <= 65536 or K <= 128 or max(M, N) * K >= (1 << 31):
+        return False
+    if K % 8 != 0 or (not tb and N % 8 != 0):
+        return M <= 128
+    if N > 49152:
+        return False
+    if tb:
+        return M <= 64
+    return M <= 16 or (M <= 32 and (N >= 16384 or K <= 4096))
+
+
+def gemm_direct_plan(M: int, N: int, K: int, tb: bool) -> Tuple[int, int, int]:
+    """(16-row fragments per wave, waves along K, segments of K) of gemm_direct.hip gemm_direct_plan."""
+    mf = 1 if M <= 16 else 2 if M <= 32 else 4
+    blocks = _cdiv(M, 16 * mf) * _cdiv(N, 64)
+    wk = 1
+    while wk < 8 and blocks * wk < 2048 and K >= 256 * wk:
+        wk *= 2
+    S = min(_cdiv(256, blocks), K // 512, 16) if blocks <= (64 if tb else 128) and K >= 2048 else 1
+    return mf, wk, S
+
+
+def _gemm_direct_launch(M: int, N: int, K: int, tb: bool) -> Tuple[HipLaunch, int]:
+    """The launch of gemm_direct.hip with the workspace its plan asks for, and its segments."""
+    mf, wk, S = gemm_direct_plan(M, N, K, tb)
+    mblocks = _cdiv(M, 16 * mf)
+    blocks = mblocks * _cdiv(N, 64) * S
+    nf = 2 if tb and blocks < 256 else 8 if not tb and mf <= 2 and blocks >= 400 and K >= 2048 else 4
+    waves = 8 if wk == 8 else 4
+    rows = 16 * (mf + nf if tb else mf)  # staged rows of 64 + 8 halves, or the wave's sums
+    lds = max(rows * 72 * 2, 16 * mf * (16 * nf + 4) * 4)
+    grid = mblocks * _cdiv(_cdiv(N, 16 * nf), waves // wk) * S
+    return HipLaunch((grid, 1, 1), (64 * waves, 1, 1), waves * lds), S
 
 
 def gemm_f32_tile_extent(M: int, N: int) -> int:
@@ -481,6 +522,8 @@ def gemm_workspace_bytes(M: int, N: int, K: int, ta: bool, tb: bool) -> int:
     neither is needed."""
     if M <= 0 or N <= 0 or K <= 0:
         return 0
+    if gemm_direct_takes(M, N, K, ta, tb):
+        return _gemm_split_bytes(M, N, gemm_direct_plan(M, N, K, tb)[2])
     return gemm_pack_bytes(M, N, K, ta, tb) + _gemm_split_bytes(M, N, gemm_split_plan(M, N, _cdiv(K, 8) * 8)[0])
 
 
