@@ -187,6 +187,75 @@ static void launch_any_grouped(const void* x, uint8_t* out, int64_t M, int64_t N
 // launch one-wave workgroups (measured 2-3% faster than four-wave ones on MI355X at 128 MiB).
 constexpr int kStreamBlock = 64;
 
+// Few long rows: a wave per row leaves most of the chip idle (33 rows of 2.9 MB ran at 0.5 TB/s), so
+// a row is cut into S segments of a wave each.  out is cleared first, in a launch of its own, and
+// a wave that finds an element stores 1: every store writes the same value, so neither the order
+// nor a partial result matters, and no workspace is needed.  kEsz and kZero as above.
+template <int kEsz, bool kZero>
+__global__ __launch_bounds__(64) void reduce_any_rows_split(const void* __restrict__ x, uint8_t* __restrict__ out,
+                                                            int64_t N, float c, int64_t seg) {
+  constexpr int kPerVec = 16 / kEsz, kUnroll = 16;
+  const int lane = threadIdx.x;
+  const int64_t row = blockIdx.y;
+  const char* rowp = reinterpret_cast<const char*>(x) + row * N * kEsz;
+  const int64_t to_edge = ((16 - (reinterpret_cast<uintptr_t>(rowp) & 15)) & 15) / kEsz;
+  const int64_t head = to_edge < N ? to_edge : N;
+  const int64_t nb = (N - head) / kPerVec, tail = N - head - nb * kPerVec;
+  const u32x4* body = reinterpret_cast<const u32x4*>(rowp + head * kEsz);
+  const auto bits = [&](uint32_t w) -> uint32_t {
+    if constexpr (kEsz == 1) return w;
+    return kZero ? (w & 0x7fffffffu) : static_cast<uint32_t>(__uint_as_float(w) != c);
+  };
+  const auto one = [&](int64_t i) -> uint32_t {
+    if constexpr (kEsz == 1) return reinterpret_cast<const uint8_t*>(rowp)[i];
+    return bits(reinterpret_cast<const uint32_t*>(rowp)[i]);
+  };
+  uint32_t acc = 0;
+  if (blockIdx.x == 0) {
+    if (lane < head) acc |= one(lane);
+    if (lane < tail) acc |= one(head + nb * kPerVec + lane);
+  }
+  const int64_t v0 = blockIdx.x * seg, v1 = v0 + seg < nb ? v0 + seg : nb;
+  for (int64_t base = v0 + lane; base < v1; base += kWave * kUnroll) {
+    u32x4 v[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {  // past the segment: its last vector again
+      const int64_t i = base + static_cast<int64_t>(u) * kWave;
+      v[u] = __builtin_nontemporal_load(body + (i < v1 ? i : v1 - 1));
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) acc |= bits(v[u].x) | bits(v[u].y) | bits(v[u].z) | bits(v[u].w);
+  }
+  acc = wave_or(acc);
+  if (lane == 0 && acc != 0u) out[row] = 1;
+}
+
+__global__ __launch_bounds__(256) void clear_u8(uint8_t* __restrict__ out, int64_t M) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < M) out[i] = 0;
+}
+
+// Segments of the split form for rows of `bytes` bytes: 16 KiB or more each, about kAnySplitWaves
+// waves in all; 1 where rows are many or short enough for a wave each.  us, wave per row -> split:
+// [1, 1048576] 260.6 -> 4.4, [33, 733001] 190.4 -> 18.5 (5.2 TB/s), [192, 331456] 93.0 -> 42.0 (6.1),
+// [128, 16384] 6.3 -> 5.2; past the line [512, 16384] 8.6 -> 9.0, [1024, 65536] 43.2 -> 43.8.
+constexpr int64_t kAnySplitWaves = 8192;
+static int64_t any_segments(int64_t M, int64_t bytes) {
+  if (M >= 512 || bytes < (64 << 10)) return 1;
+  const int64_t most = bytes >> 14, want = (kAnySplitWaves + M - 1) / M;
+  return most < want ? most : want;
+}
+
+template <int kEsz, bool kZero>
+static hipError_t launch_any_split(const void* x, uint8_t* out, int64_t M, int64_t N, float c, int64_t S,
+                                   hipStream_t s) {
+  clear_u8<<<dim3(static_cast<unsigned>((M + 255) / 256)), dim3(256), 0, s>>>(out, M);
+  const int64_t nb = N * kEsz / 16, seg = ((nb + S - 1) / S + 1023) / 1024 * 1024;
+  const dim3 grid(static_cast<unsigned>((nb + seg - 1) / seg), static_cast<unsigned>(M));
+  reduce_any_rows_split<kEsz, kZero><<<grid, dim3(64), 0, s>>>(x, out, N, c, seg);
+  return hipGetLastError();
+}
+
 hipError_t launch_reduce_any_rows_f32(const float* x, uint8_t* out, int64_t M, int64_t N, float c, hipStream_t s) {
   if (M == 0) return hipSuccess;
   if (M > 0x7fffffffLL) return hipErrorInvalidValue;  // one workgroup per row
@@ -194,11 +263,15 @@ hipError_t launch_reduce_any_rows_f32(const float* x, uint8_t* out, int64_t M, i
   // 16-byte loads over each row's aligned body whenever x is 4-byte aligned (any N)
   const bool vec = (reinterpret_cast<uintptr_t>(x) & 3) == 0;
   const int g = vec ? any_group_lanes(4 * N, 2) : 0;  // f32: a head and tail of at most 3 elements
+  const int64_t S = vec ? any_segments(M, 4 * N) : 1;
   if (g > 0) {  // short rows: several per wave
     if (c == 0.0f)
       launch_any_grouped<4, true>(x, out, M, N, c, g, s);
     else
       launch_any_grouped<4, false>(x, out, M, N, c, g, s);
+  } else if (S > 1) {
+    return c == 0.0f ? launch_any_split<4, true>(x, out, M, N, c, S, s)
+                     : launch_any_split<4, false>(x, out, M, N, c, S, s);
   } else if (!vec) {
     reduce_any_rows_f32_scalar<<<grid, block, 0, s>>>(x, out, M, N, c);
   } else if (c == 0.0f) {
@@ -220,8 +293,11 @@ hipError_t launch_reduce_any_rows_u8(const uint8_t* x, uint8_t* out, int64_t M, 
   if (M > 0x7fffffffLL) return hipErrorInvalidValue;  // one workgroup per row in the vector form
   const dim3 grid(static_cast<unsigned>(M)), block(kStreamBlock);
   const int g = any_group_lanes(N, 4);  // u8: a head and tail of up to 15 bytes over the group's lanes
+  const int64_t S = any_segments(M, N);
   if (g > 0)  // short rows: several per wave
     launch_any_grouped<1, false>(x, out, M, N, 0.0f, g, s);
+  else if (S > 1)
+    return launch_any_split<1, false>(x, out, M, N, 0.0f, S, s);
   else if (N / 16 >= kWave * 16)
     reduce_any_rows_u8_vec<16><<<grid, block, 0, s>>>(x, out, M, N);
   else

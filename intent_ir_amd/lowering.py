@@ -559,7 +559,12 @@ def _match_reduce_any(c: _Ctx) -> Optional[HipLoweredKernel]:
     # rows of at most 64 16-byte vectors: g lanes per row (about two vectors each; at least 2 lanes
     # for f32, 4 for bool), 256-thread workgroups; longer rows a one-wave workgroup each
     nvec = N // 4 if kid == "ihip_reduce_any_rows_f32" else N // 16
-    if nvec <= 64:
+    # few long rows (rows.hip any_segments): a wave per segment of a row, after a launch that clears out
+    if M < 512 and nvec >= 4096:
+        S = min(nvec >> 10, max(1, _cdiv(8192, max(1, M))))
+        seg = _cdiv(_cdiv(nvec, S), 1024) * 1024
+        launch = HipLaunch((_cdiv(nvec, seg), max(1, M), 1), (64, 1, 1), 0)
+    elif nvec <= 64:
         g = 2 if kid == "ihip_reduce_any_rows_f32" else 4
         while g < 32 and 2 * g < nvec:
             g *= 2
@@ -885,7 +890,8 @@ def _match_gelu_axpy(c: _Ctx) -> Optional[HipLoweredKernel]:
         launch = HipLaunch((max(1, _cdiv(N // 8, lanes)), max(1, min(65535, _cdiv(M, 8 * (256 // lanes)))), 1),
                            (256, 1, 1), 0)
     else:
-        launch = HipLaunch((max(1, min(65536, _cdiv(M * N, 256))), 1, 1), (256, 1, 1), 0)
+        per = 8192 if N >= 8 and M * N < (1 << 31) - (1 << 13) else 256  # runs of 8 elements, or one a thread
+        launch = HipLaunch((max(1, min(65536, _cdiv(M * N, per))), 1, 1), (256, 1, 1), 0)
     return HipLoweredKernel(c.fn.name, "ihip_bias_gelu_tanh_axpy_bf16", c.io([x, bias, oname]), launch, [oname],
                             dict(c.b), (("tensor", x), ("tensor", bias), ("tensor", oname), ("i64", M), ("i64", N),
                                         ("f32", float(env["alpha"][1]))))
