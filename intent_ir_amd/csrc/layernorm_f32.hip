@@ -8,12 +8,13 @@
 // below are compiled with contraction off), so y differs from numpy's only through the order
 // in which the two row sums are accumulated.
 //
-// Forms, the first two reading x from HBM once with the row held in registers:
+// Forms, all but the last reading x from HBM once with the row held in registers:
+//  * 4 <= N <= 256: 2-64 lanes per row, one vector each (layernorm_rows_f32_grouped);
 //  * N <= 4099: a wave per row (kVpl 16-byte vectors per lane), 4 rows per 256-thread workgroup
 //    with w and b staged in LDS once per workgroup (instead of once per row from L2);
 //  * 4099 < N <= 65539: kW waves per row, the wave sums exchanged through LDS and folded in a
 //    fixed order, w and b from L2;
-//    both come twice: kU = false for N % 4 == 0 and 16-byte aligned tensors; kU = true for rows
+//    these two come twice: kU = false for N % 4 == 0 and 16-byte aligned tensors; kU = true for rows
 //    that start at any 4-byte boundary (odd N, unaligned views): the same 16-byte accesses, of
 //    which gfx950 asks 4-byte alignment only, from the row's own start, and the last N % 4
 //    elements on the row's first lanes;
@@ -111,6 +112,56 @@ __global__ __launch_bounds__(64 * kLn32Rows) void layernorm_rows_f32_wave(
   if (live && lane == 0) {
     if (mean_out != nullptr) mean_out[row] = mean;
     if (rstd_out != nullptr) rstd_out[row] = rstd;
+  }
+}
+
+// Short rows (4 <= N <= 4 G): G lanes per row, one vector each, kR rows per group with every load
+// issued before the first is used, any 4-byte boundary.  The row's last vector starts 4 before its
+// end: the elements it shares with the one before it (the first `dup`) are left out of the sums and
+// stored twice with the same value.
+template <int G, int kR>
+__global__ __launch_bounds__(256) void layernorm_rows_f32_grouped(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y,
+    float* __restrict__ mean_out, float* __restrict__ rstd_out, int64_t M, int N, float eps) {
+  const int lig = threadIdx.x & (G - 1);
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * (256 / G) * kR + threadIdx.x / G;
+  const bool in = 4 * lig < N;  // lanes past the row hold its last vector and leave all of it out
+  const int start = 4 * lig < N - 4 ? 4 * lig : N - 4, dup = in ? 4 * lig - start : 4;
+  f32x4 xv[kR];
+#pragma unroll
+  for (int rr = 0; rr < kR; ++rr) {
+    const int64_t row = row0 + rr * (256 / G);
+    xv[rr] = ln32_load<true>(x + (row < M ? row : M - 1) * N + start);
+  }
+  const f32x4 wv = ln32_load_wb<true>(w + start), bv = ln32_load_wb<true>(b + start);
+#pragma unroll
+  for (int rr = 0; rr < kR; ++rr) {
+    const int64_t row = row0 + rr * (256 / G);
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += j >= dup ? xv[rr][j] : 0.f;
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, kWave);
+    const float mean = s / static_cast<float>(N);
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float d = xv[rr][j] - mean;
+      q += j >= dup ? d * d : 0.f;
+    }
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1) q += __shfl_xor(q, off, kWave);
+    const float rstd = 1.0f / sqrtf(q / static_cast<float>(N) + eps);
+    if (row < M) {
+      f32x4 o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = ((xv[rr][j] - mean) * rstd) * wv[j] + bv[j];
+      if (in) ln32_store<true>(y + row * N + start, o);
+      if (lig == 0) {
+        if (mean_out != nullptr) mean_out[row] = mean;
+        if (rstd_out != nullptr) rstd_out[row] = rstd;
+      }
+    }
   }
 }
 
@@ -213,6 +264,22 @@ static void launch_ln32_wave(const float* x, const float* w, const float* b, flo
       x, w, b, y, mean, rstd, M, n4, N, eps);
 }
 
+// Two rows per group, or one where that would leave fewer than 1024 workgroups ([768, 128]: 2.8
+// against 3.4 us).  us, wave per row (aligned) or three passes (other N) -> grouped: [400000, 16] 89.1
+// -> 11.7, [100000, 128] 31.0 -> 20.2, [100000, 256] 39.7 -> 36.5, [205114, 75] 249.4 -> 27.7 (four rows
+// 26.1), [1000000, 17] 1069 -> 29.8, [242880, 201] 343.6 -> 71.8 (four rows 74.6).
+template <int G>
+static void launch_ln32_grouped(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
+                                int64_t M, int N, float eps, hipStream_t s) {
+  const int64_t rows = 256 / G, two = (M + 2 * rows - 1) / (2 * rows);
+  if (two >= 1024)
+    layernorm_rows_f32_grouped<G, 2><<<dim3(static_cast<unsigned>(two)), dim3(256), 0, s>>>(x, w, b, y, mean, rstd, M,
+                                                                                           N, eps);
+  else
+    layernorm_rows_f32_grouped<G, 1><<<dim3(static_cast<unsigned>((M + rows - 1) / rows)), dim3(256), 0, s>>>(
+        x, w, b, y, mean, rstd, M, N, eps);
+}
+
 template <int kW, bool kU>
 static void launch_ln32_multi(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
                               int64_t M, int n4, int N, float eps, hipStream_t s) {
@@ -224,8 +291,17 @@ static void launch_ln32_multi(const float* x, const float* w, const float* b, fl
 template <bool kU>
 static void launch_ln32_held(const float* x, const float* w, const float* b, float* y, float* mean, float* rstd,
                              int64_t M, int N, float eps, hipStream_t s) {
-  const int n4 = N / 4;
-  if (n4 <= 64) launch_ln32_wave<1, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  const int n4 = N / 4, nv = (N + 3) / 4;
+  if (N >= 4 && nv <= 64) {
+    if (nv <= 2) launch_ln32_grouped<2>(x, w, b, y, mean, rstd, M, N, eps, s);
+    else if (nv <= 4) launch_ln32_grouped<4>(x, w, b, y, mean, rstd, M, N, eps, s);
+    else if (nv <= 8) launch_ln32_grouped<8>(x, w, b, y, mean, rstd, M, N, eps, s);
+    else if (nv <= 16) launch_ln32_grouped<16>(x, w, b, y, mean, rstd, M, N, eps, s);
+    else if (nv <= 32) launch_ln32_grouped<32>(x, w, b, y, mean, rstd, M, N, eps, s);
+    else launch_ln32_grouped<64>(x, w, b, y, mean, rstd, M, N, eps, s);
+    return;
+  }
+  if (n4 <= 64) launch_ln32_wave<1, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);  // N < 4, or 257-259
   else if (n4 <= 128) launch_ln32_wave<2, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
   else if (n4 <= 256) launch_ln32_wave<4, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
   else if (n4 <= 512) launch_ln32_wave<8, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);

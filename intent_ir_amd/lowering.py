@@ -847,11 +847,15 @@ def _match_layernorm(c: _Ctx) -> Optional[HipLoweredKernel]:
 
 
 def _layernorm_f32_launch(M: int, N: int) -> HipLaunch:
-    """The launch ihip_layernorm_rows_f32 plans (layernorm_f32.hip): up to 1024 whole 16-byte
-    vectors per row: a wave per row, 4 rows per 256-thread workgroup, w and b staged in LDS; up
-    to 16384: 2-16 waves per row, one row per workgroup; otherwise a 256-thread workgroup per
-    row."""
+    """The launch ihip_layernorm_rows_f32 plans (layernorm_f32.hip): rows of 4 to 256 elements: 2-64
+    lanes each, two rows (one in short grids) per lane group; up to 1024 whole 16-byte vectors per
+    row: a wave per row, 4 rows per 256-thread workgroup, w and b staged in LDS; up to 16384: 2-16
+    waves per row, one row per workgroup; otherwise a 256-thread workgroup per row."""
     n4 = N // 4
+    if 4 <= N <= 256:
+        g = next(v for v in (2, 4, 8, 16, 32, 64) if _cdiv(N, 4) <= v)
+        two = _cdiv(M * g, 512)
+        return HipLaunch((max(1, two if two >= 1024 else _cdiv(M * g, 256)), 1, 1), (256, 1, 1), 0)
     if N > 0 and n4 <= 1024:
         kvpl = next(v for v in (1, 2, 4, 8, 16) if n4 <= 64 * v)
         return HipLaunch((max(1, _cdiv(M, 4)), 1, 1), (256, 1, 1), 2 * 16 * 64 * kvpl)

@@ -16,6 +16,34 @@ pytestmark = pytest.mark.gpu
 P = ctypes.c_void_p
 
 
+@pytest.mark.parametrize("M,N", [(300001, 4), (270000, 7), (140001, 16), (70000, 33), (66003, 64), (40001, 101),
+                                 (9001, 129), (8200, 255), (8193, 256)])
+def test_layernorm_f32_many_short_rows(hip, M, N):
+    """Two rows per lane group (grids of 1024 workgroups and more): every row against float64."""
+    import torch
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+    x = torch.randn((M, N), generator=g, device="cuda") + 1.0
+    w, b = 1 + 0.1 * torch.randn(N, generator=g, device="cuda"), 0.1 * torch.randn(N, generator=g, device="cuda")
+    y = torch.full((M * N + 16,), 7.0, device="cuda")
+    mean, rstd = torch.empty(M, device="cuda"), torch.empty(M, device="cuda")
+    print(f"[case] layernorm f32 short rows M={M} N={N}", flush=True)
+    st = hip.ihip_layernorm_rows_f32(P(x.data_ptr()), P(w.data_ptr()), P(b.data_ptr()), P(y.data_ptr()),
+                                     P(mean.data_ptr()), P(rstd.data_ptr()), M, N, ctypes.c_float(1e-5),
+                                     P(torch.cuda.current_stream().cuda_stream))
+    assert st == 0, hip.ihip_last_error().decode()
+    xd = x.double()
+    m = xd.mean(dim=1, keepdim=True)
+    r = 1.0 / torch.sqrt(((xd - m) ** 2).mean(dim=1, keepdim=True) + 1e-5)
+    # d = x - mean carries 2^-22 of |x| + |mean|, times rstd (short rows can be nearly constant)
+    bound = 1e-5 + 1e-6 * (xd.abs() + m.abs() + 1) * r * (1 + (xd - m).abs() * r * r)
+    assert (((y[:M * N].view(M, N).double() - ((xd - m) * r * w.double() + b.double())).abs()) <= bound).all()
+    assert ((mean.double() - m[:, 0]).abs() <= 1e-6 * (1 + m[:, 0].abs())).all()
+    assert ((rstd.double() - r[:, 0]).abs() <= 1e-5 * r[:, 0] * (1 + r[:, 0])).all()
+    assert (y[M * N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 7, 255, 256, 257, 259, 511, 515, 1023, 1027, 2049, 2051, 4095, 4097, 4099,
                                4100, 4101, 8191, 8195, 16387, 32771, 65537, 65539, 65540])
 @pytest.mark.parametrize("ox,ow,ob,oy", [(0, 0, 0, 0), (1, 2, 3, 0), (0, 1, 0, 3), (3, 0, 2, 1)])
