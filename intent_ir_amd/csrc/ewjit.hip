@@ -869,7 +869,7 @@ struct JitEntry {
 };
 
 std::mutex g_jit_mu;
-std::unordered_map<std::string, JitEntry> g_jit;  // key: generated source
+std::unordered_map<std::string, JitEntry> g_jit;  // key: JitForm::key()
 
 void compile(const std::string& src, JitEntry& e) {
   hiprtcProgram prog;
@@ -896,12 +896,54 @@ void compile(const std::string& src, JitEntry& e) {
   hiprtcDestroyProgram(&prog);
 }
 
-// Cache entry of a source, compiled on first request (caller holds g_jit_mu).
-JitEntry& entry(const std::string& src) {
-  auto it = g_jit.find(src);
+// Everything the generated source depends on: the program, the operand types and access forms.
+struct JitForm {
+  const ihip_ew_instr* code = nullptr;
+  int n_code = 0, n_inputs = 0, n_outputs = 0;
+  int in_dt[IHIP_EW_NATIVE_MAX_INPUTS] = {}, out_dt[IHIP_EW_NATIVE_MAX_OUTPUTS] = {};
+  char in_kind[IHIP_EW_NATIVE_MAX_INPUTS + 1] = {}, out_kind[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = {};
+  uint32_t rowinv = 0;
+  bool flat = false;
+
+  std::string source() const {
+    return flat ? ew_jit_source_flat(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind)
+                : ew_jit_source(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind, out_kind, rowinv);
+  }
+
+  // The same, as the cache's key: a launch looks its code up by this and writes no source (that
+  // took 6-8 us of each call).
+  std::string key() const {
+    std::string k;
+    k.reserve(16 + 9 * n_code + 2 * (n_inputs + n_outputs));
+    const auto put32 = [&](uint32_t v) { k.append(reinterpret_cast<const char*>(&v), sizeof v); };
+    k.push_back(flat ? 'f' : 'r');
+    put32(static_cast<uint32_t>(n_code));
+    put32(rowinv);
+    for (int pc = 0; pc < n_code; ++pc) {
+      const ihip_ew_instr& in = code[pc];
+      for (const uint8_t b : {in.op, in.dst, in.a, in.b, in.c}) k.push_back(static_cast<char>(b));
+      put32(__builtin_bit_cast(uint32_t, in.imm));
+    }
+    for (int i = 0; i < n_inputs; ++i) {
+      k.push_back(static_cast<char>(in_dt[i]));
+      k.push_back(in_kind[i]);
+    }
+    k.push_back('>');
+    for (int i = 0; i < n_outputs; ++i) {
+      k.push_back(static_cast<char>(out_dt[i]));
+      k.push_back(out_kind[i]);
+    }
+    return k;
+  }
+};
+
+// Cache entry of a form, compiled on first request (caller holds g_jit_mu).
+JitEntry& entry(const JitForm& f) {
+  std::string k = f.key();
+  auto it = g_jit.find(k);
   if (it == g_jit.end()) {
-    it = g_jit.emplace(src, JitEntry{}).first;
-    compile(src, it->second);
+    it = g_jit.emplace(std::move(k), JitEntry{}).first;
+    compile(f.source(), it->second);
   }
   return it->second;
 }
@@ -910,10 +952,10 @@ JitEntry& entry(const std::string& src) {
 
 namespace {
 
-// Kernel arguments, generated source and grid of one launch of a validated program.
+// Kernel arguments, form and grid of one launch of a validated program.
 struct JitPlan {
   EwJitArgs a{};
-  std::string src;
+  JitForm form;
   unsigned gx = 0, gy = 0;
 };
 
@@ -930,8 +972,8 @@ struct JitPlan {
 // bf16 [100000, 200] 28.2 -> 18.0, [40000, 1040] 37.2 -> 33.0, [8192, 2600] 22.3 -> 19.2; on the
 // other side f32 [100000, 200] (78%) 29.7 -> 30.2, [60000, 512] 41.4 -> 43.5, [8192, 8192] 85.2 -> 89.0,
 // bf16 [20000, 4096] 58.6 -> 60.2.
-bool plan_flat(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inputs, int n_inputs, const int* in_dt,
-               int n_outputs, const int* out_dt, const int64_t (&shape)[4], bool vectors, int V, JitPlan& pl) {
+bool plan_flat(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inputs, int n_inputs,
+               const int64_t (&shape)[4], bool vectors, int V, JitPlan& pl) {
   EwJitArgs& a = pl.a;
   const int64_t D3 = shape[3], total = a.rows * D3;
   const int64_t wave_lanes = (a.nvec + 63) / 64 * 64, wg_lanes = (a.nvec + 255) / 256 * 256;
@@ -960,7 +1002,10 @@ bool plan_flat(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inp
   while ((int64_t(1) << l) < D3) ++l;
   a.shift = static_cast<uint32_t>(31 + l);
   a.magic = static_cast<uint32_t>(((static_cast<unsigned __int128>(1) << (31 + l)) / D3) + 1);
-  pl.src = ew_jit_source_flat(code, n_code, n_inputs, in_dt, n_outputs, out_dt, kind);
+  pl.form.flat = true;
+  for (int k = 0; k < n_inputs; ++k) pl.form.in_kind[k] = kind[k];
+  for (int k = 0; k < pl.form.n_outputs; ++k) pl.form.out_kind[k] = 'u';
+  pl.form.rowinv = 0;
   uint32_t scalars = 0;
   for (int k = 0; k < n_inputs; ++k) scalars |= kind[k] == 'b' ? 1u << k : 0u;
   const int64_t per_wg = 256 * V * static_cast<int64_t>(ew_jit_rows_per_trip(code, n_code, V, scalars));
@@ -977,7 +1022,13 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
               const ihip_ew_operand* outputs, int n_outputs, const int64_t (&shape)[4], JitPlan& pl) {
   EwJitArgs& a = pl.a;
   for (int d = 0; d < 4; ++d) a.shape[d] = shape[d];
-  int in_dt[IHIP_EW_NATIVE_MAX_INPUTS] = {}, out_dt[IHIP_EW_NATIVE_MAX_OUTPUTS] = {};
+  JitForm& f = pl.form;
+  f.code = code;
+  f.n_code = n_code;
+  f.n_inputs = n_inputs;
+  f.n_outputs = n_outputs;
+  int(&in_dt)[IHIP_EW_NATIVE_MAX_INPUTS] = f.in_dt;
+  int(&out_dt)[IHIP_EW_NATIVE_MAX_OUTPUTS] = f.out_dt;
   for (int k = 0; k < n_inputs; ++k) in_dt[k] = inputs[k].dtype;
   for (int k = 0; k < n_outputs; ++k) out_dt[k] = outputs[k].dtype;
   const int V = ew_jit_width(n_inputs, in_dt, n_outputs, out_dt);
@@ -1006,7 +1057,8 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     return shape[2] % vs == 0 && st[3] % vs == 0 && (st[0] % vs == 0 || shape[0] == 1) &&
            (st[1] % vs == 0 || shape[1] == 1) && reinterpret_cast<uintptr_t>(inputs[k].ptr) % 16 == 0;
   };
-  char in_kind[IHIP_EW_NATIVE_MAX_INPUTS + 1] = {}, out_kind[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = {};
+  char(&in_kind)[IHIP_EW_NATIVE_MAX_INPUTS + 1] = f.in_kind;
+  char(&out_kind)[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = f.out_kind;
   for (int k = 0; k < n_inputs; ++k) {
     a.in_ptr[k] = inputs[k].ptr;
     for (int d = 0; d < 4; ++d) a.in_stride[k][d] = inputs[k].stride[d];
@@ -1035,9 +1087,9 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     bool vectors = true;
     for (int k = 0; k < n_inputs; ++k) vectors &= in_kind[k] == full || in_kind[k] == 'b';
     for (int k = 0; k < n_outputs; ++k) vectors &= out_kind[k] == full;
-    if (plan_flat(code, n_code, inputs, n_inputs, in_dt, n_outputs, out_dt, shape, vectors, V, pl)) return true;
+    if (plan_flat(code, n_code, inputs, n_inputs, shape, vectors, V, pl)) return true;
   }
-  pl.src = ew_jit_source(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind, out_kind, rowinv);
+  f.rowinv = rowinv;
   if (tile_mask != 0) {  // one workgroup per 64 x 64 tile (linear id; grid-strided beyond the grid limits)
     const int64_t tx = (shape[3] + 63) / 64, ty = shape[0] * shape[1] * ((shape[2] + 63) / 64);
     pl.gx = static_cast<unsigned>(tx < 65535 ? tx : 65535);
@@ -1058,9 +1110,9 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
   return true;
 }
 
-bool compile_checked(const std::string& src, std::string* why) {
+bool compile_checked(const JitForm& form, std::string* why) {
   std::lock_guard<std::mutex> lock(g_jit_mu);
-  JitEntry& e = entry(src);
+  JitEntry& e = entry(form);
   if (!e.error.empty() && why) *why = e.error;
   return e.error.empty();
 }
@@ -1073,10 +1125,14 @@ bool compile_checked(const std::string& src, std::string* why) {
 bool prepare_elementwise_jit(const ihip_ew_instr* code, int n_code, int n_inputs, const int* in_dt, int n_outputs,
                              const int* out_dt, std::string* why) {
   const char w = ew_jit_width(n_inputs, in_dt, n_outputs, out_dt) == 8 ? '8' : '4';
-  char in_kind[IHIP_EW_NATIVE_MAX_INPUTS + 1] = {}, out_kind[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = {};
-  for (int k = 0; k < n_inputs; ++k) in_kind[k] = w;
-  for (int k = 0; k < n_outputs; ++k) out_kind[k] = w;
-  return compile_checked(ew_jit_source(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind, out_kind, 0), why);
+  JitForm f;
+  f.code = code;
+  f.n_code = n_code;
+  f.n_inputs = n_inputs;
+  f.n_outputs = n_outputs;
+  for (int k = 0; k < n_inputs; ++k) f.in_dt[k] = in_dt[k], f.in_kind[k] = w;
+  for (int k = 0; k < n_outputs; ++k) f.out_dt[k] = out_dt[k], f.out_kind[k] = w;
+  return compile_checked(f, why);
 }
 
 // Compile (once) exactly the code that launch_elementwise_jit would run for these operands and
@@ -1086,7 +1142,7 @@ bool prepare_elementwise_jit_operands(const ihip_ew_instr* code, int n_code, con
                                       const int64_t (&shape)[4], std::string* why) {
   JitPlan pl;
   if (!plan_jit(code, n_code, inputs, n_inputs, outputs, n_outputs, shape, pl)) return true;
-  return compile_checked(pl.src, why);
+  return compile_checked(pl.form, why);
 }
 
 // The source that launch_elementwise_jit would compile for these operands and shape ("" when
@@ -1095,7 +1151,7 @@ std::string source_elementwise_jit_operands(const ihip_ew_instr* code, int n_cod
                                             int n_inputs, const ihip_ew_operand* outputs, int n_outputs,
                                             const int64_t (&shape)[4]) {
   JitPlan pl;
-  return plan_jit(code, n_code, inputs, n_inputs, outputs, n_outputs, shape, pl) ? pl.src : std::string();
+  return plan_jit(code, n_code, inputs, n_inputs, outputs, n_outputs, shape, pl) ? pl.form.source() : std::string();
 }
 
 // Launch the specialised kernel of a validated program; compiles on first use.  Returns
@@ -1111,7 +1167,7 @@ hipError_t launch_elementwise_jit(const ihip_ew_instr* code, int n_code, const i
   hipFunction_t fn = nullptr;
   {
     std::lock_guard<std::mutex> lock(g_jit_mu);
-    JitEntry& e = entry(pl.src);
+    JitEntry& e = entry(pl.form);
     if (!e.error.empty()) {
       if (why) *why = e.error;
       return hipErrorNotSupported;

@@ -68,6 +68,10 @@ class HipLoweredKernel:
     # ihip_elementwise_program.  io_spec["hip_call"] holds the same plan as JSON.
     call_args: Tuple[Tuple[str, Any], ...] = field(default_factory=tuple)
 
+    def __getstate__(self):
+        """The fields only: the runtime's call plan (runtime._CallPlan) is rebuilt at the first launch."""
+        return {k: v for k, v in self.__dict__.items() if k != "_call_plan"}
+
 
 def _cdiv(a: int, b: int) -> int:
     return -(-a // b)

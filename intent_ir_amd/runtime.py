@@ -211,41 +211,77 @@ def _check_buffer(name: str, t, dtype: str, shape: Sequence[int]) -> None:
         raise HipRuntimeError(f"{name}: tensor must be contiguous")
 
 
-def _ctype_args(call_args: Iterable[Tuple[str, Any]], buffers: Mapping[str, Any], keep: list,
-                dtypes: Optional[Mapping[str, str]] = None, stream=None):
-    """ctypes arguments of a lowered call.  A workspace is a fresh torch allocation marked as used
-    by ``stream`` (record_stream), so the caching allocator does not hand it out again before the
-    kernels reading it have run: no host synchronisation is needed."""
-    out = []
-    for kind, v in call_args:
-        if kind == "ew_program":
-            args = ew_program_args(v, {n: buffers[n].data_ptr() for n in buffers}, dtypes or {})
-            keep.append(args.pop())  # keep the ctypes arrays alive through the call
-            out.extend(args)
-        elif kind == "tensor":
-            out.append(_P(buffers[v].data_ptr()))
-        elif kind == "i64":
-            out.append(_I64(int(v)))
-        elif kind == "i32":
-            out.append(_I32(int(v)))
-        elif kind == "f32":
-            out.append(_F32(float(v)))
-        elif kind == "null":
-            out.append(_P(None))
-        elif kind == "workspace":
-            torch = _torch()
-            t = torch.empty(max(1, int(v)), dtype=torch.uint8, device="cuda")
-            if stream is not None:
-                t.record_stream(stream)
-            keep.append(t)
-            out.extend([_P(t.data_ptr()), _I64(int(v))])
-        else:
-            raise HipRuntimeError(f"unknown call argument kind {kind}")
-    return out
-
-
 def tensor_shapes(io_spec: Mapping[str, Any], bindings: Mapping[str, Any]) -> Dict[str, Tuple[int, ...]]:
     return {n: tuple(resolve_dim(d, bindings) for d in spec["shape"]) for n, spec in io_spec["tensors"].items()}
+
+
+class _CallPlan:
+    """What every launch of one lowered kernel shares, worked out once: the tensors' torch dtypes and
+    bound shapes, the entry point, and the C arguments that are not pointers.  Nothing of a buffer is
+    kept, and nothing here is written after it is built, so threads may share it."""
+
+    __slots__ = ("io_spec", "bindings", "bound", "call_args", "kernel_id", "tensors", "fn", "args", "ptr_slots",
+                 "workspaces", "program")
+
+    def __init__(self, lowered) -> None:
+        self.io_spec, self.bindings = lowered.io_spec, lowered.bindings
+        self.bound = dict(lowered.bindings)
+        self.call_args, self.kernel_id = lowered.call_args, lowered.kernel_id
+        shapes = tensor_shapes(lowered.io_spec, lowered.bindings)
+        self.tensors = tuple((n, spec["dtype"], torch_dtype(spec["dtype"]), shapes[n])
+                             for n, spec in lowered.io_spec["tensors"].items())
+        self.fn = getattr(load_library(), lowered.kernel_id)
+        args: list = []
+        slots, workspaces = [], []
+        self.program = None
+        for kind, v in lowered.call_args:
+            if kind == "tensor":
+                slots.append((len(args), v))
+                args.append(None)
+            elif kind == "workspace":
+                workspaces.append((len(args), int(v)))
+                args += [None, int(v)]
+            elif kind == "ew_program":
+                dtypes = {n: spec["dtype"] for n, spec in lowered.io_spec["tensors"].items()}
+                names = {n: 0 for n, _ in v.inputs} | {n: 0 for n in v.outputs}
+                prog = ew_program_args(v, names, dtypes)
+                code, ins, outs, shape = prog.pop()
+                self.program = (code, type(ins), bytes(ins), tuple(n for n, _ in v.inputs), type(outs), bytes(outs),
+                                tuple(v.outputs), shape, len(args))
+                args += [code, len(v.code), None, len(v.inputs), None, len(v.outputs), shape, len(v.shape)]
+            elif kind in ("i64", "i32"):
+                args.append(int(v))
+            elif kind == "f32":
+                args.append(float(v))
+            elif kind == "null":
+                args.append(None)
+            else:
+                raise HipRuntimeError(f"unknown call argument kind {kind}")
+        args.append(None)  # the stream
+        self.args, self.ptr_slots, self.workspaces = args, tuple(slots), tuple(workspaces)
+
+    def of(self, lowered) -> bool:
+        return (self.io_spec is lowered.io_spec and self.call_args is lowered.call_args
+                and self.kernel_id == lowered.kernel_id and self.bindings is lowered.bindings
+                and self.bound == lowered.bindings)
+
+
+def _call_plan(lowered) -> _CallPlan:
+    """The kernel's plan: kept in the lowered object itself (and rebuilt if its parts were replaced)."""
+    plan = lowered.__dict__.get("_call_plan")
+    if plan is None or not plan.of(lowered):
+        _torch()  # no device: that error first
+        plan = _CallPlan(lowered)
+        lowered.__dict__["_call_plan"] = plan
+    return plan
+
+
+def _raw_stream(torch) -> int:
+    """hipStream_t of torch's current stream on the current device."""
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:  # a torch without the raw accessors
+        return torch.cuda.current_stream().cuda_stream
 
 
 def launch_lowered(lowered, buffers: Mapping[str, Any], stream=None) -> None:
@@ -253,18 +289,48 @@ def launch_lowered(lowered, buffers: Mapping[str, Any], stream=None) -> None:
 
     ``buffers`` maps every tensor of ``lowered.io_spec`` to a contiguous device
     tensor of the declared dtype and bound shape; ``stream`` is a torch stream or
-    None for torch's current stream."""
-    torch = _torch()
-    shapes = tensor_shapes(lowered.io_spec, lowered.bindings)
-    for n, spec in lowered.io_spec["tensors"].items():
+    None for torch's current stream.  The host's share of a call is checking the
+    buffers and passing their addresses; the rest comes from the kernel's plan."""
+    try:
+        import torch  # noqa: PLC0415
+    except ImportError:
+        torch = _torch()  # raises
+    plan = _call_plan(lowered)
+    Tensor = torch.Tensor
+    ptrs = {}
+    for n, dt, tdt, shape in plan.tensors:
+        t = buffers.get(n)
+        if (isinstance(t, Tensor) and t.is_cuda and t.dtype is tdt and t.shape == shape and t.is_contiguous()):
+            ptrs[n] = t.data_ptr()
+            continue
+        _torch()
         if n not in buffers:
             raise HipRuntimeError(f"missing buffer for {n}")
-        _check_buffer(n, buffers[n], spec["dtype"], shapes[n])
-    s = stream if stream is not None else torch.cuda.current_stream()
-    keep: list = []  # host-side ctypes arrays of an element-wise program (copied at launch)
-    dtypes = {n: spec["dtype"] for n, spec in lowered.io_spec["tensors"].items()}
-    args = _ctype_args(lowered.call_args, buffers, keep, dtypes, s)
-    call(lowered.kernel_id, *args, _P(s.cuda_stream))
+        _check_buffer(n, t, dt, shape)  # raises, unless t is the bound shape in another arrangement of its axes
+        ptrs[n] = t.data_ptr()
+    args = plan.args.copy()
+    for i, n in plan.ptr_slots:
+        args[i] = ptrs[n]
+    keep = []
+    for i, nbytes in plan.workspaces:
+        t = torch.empty(max(1, nbytes), dtype=torch.uint8, device="cuda")
+        if stream is not None:  # allocated on the current stream, used on this one
+            t.record_stream(stream)
+        keep.append(t)
+        args[i] = t.data_ptr()
+    if plan.program is not None:  # operand tables of this call's own
+        _, in_t, in_b, in_names, out_t, out_b, out_names, _, at = plan.program
+        ins, outs = in_t.from_buffer_copy(in_b), out_t.from_buffer_copy(out_b)
+        for i, n in enumerate(in_names):
+            ins[i].ptr = ptrs[n]
+        for i, n in enumerate(out_names):
+            outs[i].ptr = ptrs[n]
+        args[at + 2], args[at + 4] = ins, outs
+    args[-1] = stream.cuda_stream if stream is not None else _raw_stream(torch)
+    status = plan.fn(*args)
+    if status != 0:
+        msg = load_library().ihip_last_error().decode(errors="replace")
+        raise HipRuntimeError(f"{plan.kernel_id} failed (status {status}): {msg}")
 
 
 def run_hip_kernel(*, kernel_name: str, kernel_id: str, io_spec: Mapping[str, Any], launch: Any,
