@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void reduce_rows_f32(const float* __restrict__
 constexpr int kRedUnroll = 16;
 
 // Row split for rows too few to fill the GPU: S segments per row (1 = no split), so that
-// M * S workgroups of 16 waves give every CU about two, each segment at least
+// M * S workgroups of 4 or 16 waves give every CU about two, each segment at least
 // kRedSegMinVec 16-byte vectors (64 KiB).  Depends on the shape only.
 constexpr int kRedMaxSegments = 64;
 constexpr int64_t kRedSplitRows = 256;      // rows below this may split (fewer rows than CUs)
@@ -528,8 +528,18 @@ static void launch_reduce_rows(const float* x, float* out, int64_t M, int64_t N,
   const int64_t n4 = N / 4;
   const dim3 grid(static_cast<unsigned>(M));
   if (S > 1 && part != nullptr) {  // few long rows split over S workgroups each, then combined
-    reduce_rows_f32_vec<kKind, 16, 8, 4, true><<<dim3(static_cast<unsigned>(M * S)), dim3(1024), 0, s>>>(
-        x, out, M, N, scale, S, part);
+    // Workgroups of 4 waves where they are about two per CU, of 16 where they are fewer or the CUs
+    // get unequal numbers of them.  us, 16 waves with 8 loads in flight per lane (before), with 4, and
+    // 4 waves with 8: [64, 1048576] 49.0, 45.7, 42.6 (6.3 TB/s); [16, 4000000] 44.7, 44.3, 43.2;
+    // [200, 300001] (600 workgroups) 45.5, 45.4, 46.2; [200, 40000] (400) 9.7, 9.7, 10.0; [1, 1048576]
+    // (64) 5.5, 5.5, 5.9.  8 partial sums per lane keep the error where it was (rms over 30 draws of
+    // [64, 1048576] uniform terms: 4.4e-8 before, 4.2e-8).
+    if (M * S >= 448 && M * S <= 512)
+      reduce_rows_f32_vec<kKind, 4, 8, 8, true><<<dim3(static_cast<unsigned>(M * S)), dim3(256), 0, s>>>(
+          x, out, M, N, scale, S, part);
+    else
+      reduce_rows_f32_vec<kKind, 16, 4, 4, true><<<dim3(static_cast<unsigned>(M * S)), dim3(1024), 0, s>>>(
+          x, out, M, N, scale, S, part);
     reduce_rows_combine<kKind><<<dim3(static_cast<unsigned>((M + 3) / 4)), dim3(256), 0, s>>>(part, out, M, S, scale);
   } else if (n4 <= 2 * kWave) {  // short rows: several per wave
     launch_reduce_grouped<kKind>(x, out, M, N, scale, s);

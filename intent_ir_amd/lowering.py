@@ -932,8 +932,9 @@ def _match_row_reduce(c: _Ctx) -> Optional[HipLoweredKernel]:
     if scale is not None:  # out = sum * scale: the _ex entry, with the split workspace when the rule splits
         kid = "ihip_reduce_rows_f32_ex"
         args += (("f32", scale),) + ((("workspace", 4 * M * segs),) if segs > 1 else (("null", None), ("i64", 0)))
-    if segs > 1:  # rows too few for the CUs: S workgroups of 16 waves per row, partials in a workspace
-        launch = HipLaunch((M * segs, 1, 1), (1024, 1, 1), 64)
+    if segs > 1:  # rows too few for the CUs: S workgroups of 4 or 16 waves per row, partials in a workspace
+        w = 4 if 448 <= M * segs <= 512 else 16
+        launch = HipLaunch((M * segs, 1, 1), (64 * w, 1, 1), 4 * w)
         if scale is None:
             kid, args = "ihip_reduce_rows_f32_ws", args + (("workspace", 4 * M * segs),)
         return HipLoweredKernel(c.fn.name, kid, c.io([x, oname]), launch, [oname], dict(c.b), args)
