@@ -198,6 +198,17 @@ int ihip_gemm_bf16_bias_relu(const uint16_t* A, const uint16_t* B, const float* 
 int ihip_gemm_f32_bias_relu(const float* A, const float* B, const float* bias, float* C, int64_t M, int64_t N,
                             int64_t K, int transpose_a, int transpose_b, int relu, int tile, void* stream);
 
+/* The same with a caller-owned workspace (16-byte aligned, ihip_gemm_f32_workspace_size bytes): with
+ * the automatic tile, a product of too few C tiles to fill the GPU is cut along K, its partial
+ * sums go to the workspace and a second launch adds them in order.  Deterministic; C differs from
+ * the unsplit one by the f32 summation order only.  A NULL or smaller workspace: no split. */
+int ihip_gemm_f32_bias_relu_ws(const float* A, const float* B, const float* bias, float* C, int64_t M, int64_t N,
+                               int64_t K, int transpose_a, int transpose_b, int relu, int tile, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
+/* Bytes of that workspace for a shape, 0 where K is not split. */
+int64_t ihip_gemm_f32_workspace_size(int64_t M, int64_t N, int64_t K);
+
 /* The same with matmul's transpose flags (verify/interpreter.py:507-520): when transpose_a,
  * A is given as [K, M] and the product uses its transpose; when transpose_b, B is given as
  * [N, K].  Every layout runs the same MFMA schedule and accumulates in the same order, so a

@@ -31,7 +31,8 @@ hipError_t launch_layernorm_rows_f16(const uint16_t*, const uint16_t*, const uin
 hipError_t launch_layernorm_rows_f32(const float*, const float*, const float*, float*, float*, float*, int64_t, int64_t,
                                      float, hipStream_t);
 hipError_t launch_gemm_f32_bias_relu(const float*, const float*, const float*, float*, int64_t, int64_t, int64_t, bool,
-                                     bool, int, int, hipStream_t);
+                                     bool, int, int, void*, int64_t, hipStream_t);
+int64_t gemm_f32_workspace_bytes(int64_t, int64_t, int64_t);
 hipError_t launch_bias_gelu_axpy_bf16(const uint16_t*, const uint16_t*, uint16_t*, int64_t, int64_t, float,
                                       hipStream_t);
 hipError_t launch_gather2d_f32(const float*, const int32_t*, const int32_t*, float*, int64_t, int64_t, int64_t, float,
@@ -388,16 +389,29 @@ int ihip_gemm_bf16_bias_relu_ex(const uint16_t* A, const uint16_t* B, const floa
                 "gemm_bf16_bias_relu");
 }
 
+int64_t ihip_gemm_f32_workspace_size(int64_t M, int64_t N, int64_t K) {
+  if (numel2(M, K) < 0 || numel2(K, N) < 0 || numel2(M, N) < 0) return 0;
+  return ihip::gemm_f32_workspace_bytes(M, N, K);
+}
+
 int ihip_gemm_f32_bias_relu(const float* A, const float* B, const float* bias, float* C, int64_t M, int64_t N,
                             int64_t K, int transpose_a, int transpose_b, int relu, int tile, void* stream) {
+  return ihip_gemm_f32_bias_relu_ws(A, B, bias, C, M, N, K, transpose_a, transpose_b, relu, tile, nullptr, 0, stream);
+}
+
+int ihip_gemm_f32_bias_relu_ws(const float* A, const float* B, const float* bias, float* C, int64_t M, int64_t N,
+                               int64_t K, int transpose_a, int transpose_b, int relu, int tile, void* workspace,
+                               int64_t workspace_bytes, void* stream) {
   IHIP_REQUIRE(numel2(M, K) >= 0 && numel2(K, N) >= 0 && numel2(M, N) >= 0,
                "gemm_f32_bias_relu: invalid shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
   IHIP_REQUIRE(M == 0 || N == 0 || C != nullptr, "gemm_f32_bias_relu: C is null");
   IHIP_REQUIRE(M == 0 || N == 0 || K == 0 || (A != nullptr && B != nullptr), "gemm_f32_bias_relu: A or B is null");
   IHIP_REQUIRE(tile == 0 || tile == 64 || tile == 128, "gemm_f32_bias_relu: tile %d is not 0 (automatic), 64 or 128",
                tile);
+  IHIP_REQUIRE(workspace_bytes >= 0 && (workspace_bytes == 0 || workspace != nullptr),
+               "gemm_f32_bias_relu: workspace of %lld bytes at a null pointer", (long long)workspace_bytes);
   return finish(ihip::launch_gemm_f32_bias_relu(A, B, bias, C, M, N, K, transpose_a != 0, transpose_b != 0, relu, tile,
-                                                static_cast<hipStream_t>(stream)),
+                                                workspace, workspace_bytes, static_cast<hipStream_t>(stream)),
                 "gemm_f32_bias_relu");
 }
 

@@ -397,6 +397,26 @@ def gemm_f32_tile_extent(M: int, N: int) -> int:
     return 64 if _cdiv(M, 128) * _cdiv(N, 128) < 256 else 128
 
 
+def gemm_f32_split_plan(M: int, N: int, K: int) -> Tuple[int, int]:
+    """(S, k per segment) of gemm_f32.hip f32_split_plan with the automatic tile."""
+    best = (1, K)
+    if M <= 0 or N <= 0 or gemm_f32_tile_extent(M, N) != 64:
+        return best
+    tiles, ldp = _cdiv(M, 64) * _cdiv(N, 64), _cdiv(N, 4) * 4
+
+    def tiles_ns(wgs: int, k: int) -> int:
+        return (wgs // 1024 * 95 + (0, 34, 50, 73, 95)[_cdiv(wgs % 1024, 256)]) * k
+
+    best_ns = tiles_ns(tiles, K)
+    for S in range(2, min(32, K // 128) + 1):
+        kseg = _cdiv(_cdiv(K, S), 32) * 32
+        segs = _cdiv(K, kseg)
+        ns = tiles_ns(tiles * segs, kseg) + 4000 + segs * M * ldp * 8 // 6000
+        if ns < best_ns:
+            best, best_ns = (segs, kseg), ns
+    return best
+
+
 def _gemm_f32(c: "_Ctx", a: str, b: str, bias: Optional[str], oname: str, M: int, N: int, K: int, ta: bool,
               tb: bool, relu: bool, names: List[str]) -> HipLoweredKernel:
     """The reference's own matmul IR (f32 A, B, C: intentir_to_cuda.py:537-985, with the bias +
@@ -408,6 +428,11 @@ def _gemm_f32(c: "_Ctx", a: str, b: str, bias: Optional[str], oname: str, M: int
     args = (("tensor", a), ("tensor", b), ("tensor", bias) if bias else ("null", None), ("tensor", oname),
             ("i64", M), ("i64", N), ("i64", K), ("i32", int(ta)), ("i32", int(tb)), ("i32", int(relu)),
             ("i32", tile))
+    S = gemm_f32_split_plan(M, N, K)[0] if tile == 0 else 1
+    if S > 1:  # too few tiles for the CUs: tiles x S workgroups, partial sums in a workspace
+        launch = HipLaunch((launch.grid[0] * S, 1, 1), (256, 1, 1), lds)
+        args += (("workspace", S * M * _cdiv(N, 4) * 16),)
+        return HipLoweredKernel(c.fn.name, "ihip_gemm_f32_bias_relu_ws", c.io(names), launch, [oname], dict(c.b), args)
     return HipLoweredKernel(c.fn.name, "ihip_gemm_f32_bias_relu", c.io(names), launch, [oname], dict(c.b), args)
 
 

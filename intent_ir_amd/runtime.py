@@ -58,6 +58,8 @@ SIGNATURES: Dict[str, Tuple[Any, Tuple[Any, ...]]] = {
     "ihip_gemm_bf16_bias_relu_t": (_I32, (_P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _P)),
     "ihip_gemm_bf16_bias_relu_ex": (_I32, (_P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _P)),
     "ihip_gemm_f32_bias_relu": (_I32, (_P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _P)),
+    "ihip_gemm_f32_bias_relu_ws": (_I32, (_P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _P, _I64, _P)),
+    "ihip_gemm_f32_workspace_size": (_I64, (_I64, _I64, _I64)),
     "ihip_gemm_workspace_size": (_I64, (_I64, _I64, _I64, _I32, _I32)),
     "ihip_gemm_bf16_bias_relu_ws": (_I32, (_P, _P, _P, _P, _I64, _I64, _I64, _I32, _I32, _I32, _I32, _P, _I64, _P)),
     "ihip_gemm_splitk_workspace_size": (_I64, (_I64, _I64, _I64, _I32)),
