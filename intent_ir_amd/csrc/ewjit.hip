@@ -156,6 +156,14 @@ template <int DT> __device__ __forceinline__ void ld4(const void* p, i64 i, floa
     v[0] = (float)(int)q.x; v[1] = (float)(int)q.y; v[2] = (float)(int)q.z; v[3] = (float)(int)q.w;
   }
 }
+// ld4 of a 32-bit operand with an ordinary load.
+template <int DT> __device__ __forceinline__ void ld4c(const void* p, i64 i, float* v) {
+  const u32x4 q = *(const u32x4*)((const u32*)p + i);
+  for (int j = 0; j < 4; ++j) {
+    const u32 w = q[j];  // __builtin_bit_cast of a vector's element would read element 0
+    v[j] = DT == 0 ? __builtin_bit_cast(float, w) : (float)(int)w;
+  }
+}
 template <int DT> __device__ __forceinline__ void st1(void* p, i64 i, float x) {
   if (DT == 0) ((float*)p)[i] = x;
   else if (DT == 1) ((u16*)p)[i] = f2h(x);
@@ -386,7 +394,7 @@ int ew_jit_width(int n_inputs, const int* in_dt, int n_outputs, const int* out_d
   return 8;
 }
 
-static bool is_tiled(char kind) { return kind == 'v' || kind == 't'; }
+static bool is_tiled(char kind) { return kind == 'v' || kind == 'V' || kind == 't'; }
 
 // Registers an instruction reads (up to 3) and the one it writes (-1 for a store).
 static int ew_reads(const ihip_ew_instr& in, int (&r)[3]) {
@@ -531,7 +539,7 @@ static std::string ew_logistic_t(const ihip_ew_instr* code, int pe, int u_reg,
 
 // Program body: the instruction list as straight-line code over r[EW_NREG][EW_V].  Inputs and
 // outputs are accessed in their form (in_kind / out_kind, see ldk); in the tiled form
-// (`tiled`) staged inputs ('v', 't') are read from their LDS tile (slot = their rank among
+// (`tiled`) staged inputs ('v', 'V', 't') are read from their LDS tile (slot = their rank among
 // the staged inputs) and the other inputs from the registers they were prefetched into.
 // preload (untiled form only): every LOAD was issued ahead into L<pc>[u] (u: the lane's row of
 // the trip; L<pc>[0] for the row-invariant inputs of `rowinv`) and becomes a register copy;
@@ -641,7 +649,8 @@ int ew_jit_rows_per_trip(const ihip_ew_instr* code, int n_code, int V, uint32_t 
 }
 
 std::string ew_jit_source(const ihip_ew_instr* code, int n_code, int n_inputs, const int* in_dt, int n_outputs,
-                          const int* out_dt, const char* in_kind, const char* out_kind, uint32_t rowinv) {
+                          const int* out_dt, const char* in_kind, const char* out_kind, uint32_t rowinv,
+                          bool wide) {
   const int V = ew_jit_width(n_inputs, in_dt, n_outputs, out_dt);
   int nreg = IHIP_EW_MAX_REGS;  // registers the program writes: r[0 .. nreg - 1]
   for (int pc = 0; pc < n_code; ++pc)
@@ -697,61 +706,63 @@ std::string ew_jit_source(const ihip_ew_instr* code, int n_code, int n_inputs, c
     return s;
   }
   // Tiled form for inputs read across their unit-stride axis (axis 2 contiguous, axis 3
-  // strided, e.g. a transpose): a workgroup takes 64 rows (axis 2) x 64 columns (axis 3).
+  // strided, e.g. a transpose): a workgroup takes T2 rows (axis 2) x T3 columns (axis 3), 64 x 64 or
+  // 128 x 32 (plan_jit).
   // Each staged input is read with consecutive threads on consecutive addresses of its axis 2
-  // (16-byte vectors for kind 'v', elements for 't') and written to an LDS tile.  Then 64/EW_V
-  // consecutive threads cover one row's 64 columns (EW_V each), so stores and the other
-  // operands' accesses stay contiguous, in 16/EW_V passes of 4*EW_V rows.  The 65-float tile
-  // pitch keeps both the staging writes and the reads conflict-free.
+  // (16-byte vectors for kinds 'v' and 'V', elements for 't') and written to an LDS tile.  Then T3/EW_V
+  // consecutive threads cover one row's T3 columns (EW_V each), so stores and the other
+  // operands' accesses stay contiguous, in 16/EW_V passes.  The tile pitch EW_P keeps the reads
+  // conflict-free, and the staging writes too (64 x 64) or two lanes to a bank (128 x 32).
   // Every global load of a tile (staging, and the other inputs for all passes) is issued
   // before the first wait: lanes outside the tensor load from a clamped, valid address, so no
   // load sits behind a branch.  Such values only reach elements that are never stored.
   // Tile order: workgroups are dispatched in order of their linear id, and EW_GROUP
-  // consecutive ids take consecutive axis-2 tiles at the same axis-3 tile.  With EW_GROUP =
-  // 64 / element size, their staging reads cover 4 KiB of each source row; measured on
-  // 8192^2 transposes: 4.9 TB/s (f32) and 4.6 TB/s (f16), against 4.3 and 3.7 with the
-  // axis-3 tiles consecutive.
+  // consecutive ids take consecutive axis-2 tiles at the same axis-3 tile, so that their staging
+  // reads cover 4 KiB of each source row (with the axis-3 tiles consecutive, 8192^2 transposes ran
+  // at 4.3 against 4.9 TB/s in f32, 3.7 against 4.6 in f16).
   int esz = 1;
   for (int k = 0; k < n_inputs; ++k)
     if (is_tiled(in_kind[k])) esz = std::max(esz, (in_dt[k] == IHIP_DT_F32 || in_dt[k] == IHIP_DT_I32) ? 4 : 2);
-  s += fmt("#define EW_NT %d\n#define EW_GROUP %d\n", nt, 64 / esz);
+  const int t2 = wide ? 128 : 64, t3 = wide ? 32 : 64;
+  s += fmt("#define EW_T2 %d\n#define EW_T3 %d\n#define EW_P %d\n", t2, t3, wide ? 130 : 65);
+  s += fmt("#define EW_NT %d\n#define EW_GROUP %d\n", nt, 4096 / (esz * t2));
   s += "extern \"C\" __global__ __launch_bounds__(256) void ihip_ew_jit(const EwJitArgs a) {\n"
-       "  __shared__ float tile[EW_NT][64][65];\n"
+       "  __shared__ float tile[EW_NT][EW_T3][EW_P];\n"
        "  const i64 D0 = a.shape[0], D1 = a.shape[1], D2 = a.shape[2], D3 = a.shape[3];\n"
-       "  const i64 T2 = (D2 + 63) / 64, ytiles = D0 * D1 * T2;\n"
-       "  const int tid = threadIdx.x, l3 = (tid % (64 / EW_V)) * EW_V;\n"
-       "  const i64 TX = (D3 + 63) / 64, ntiles = ytiles * TX;\n"
+       "  const i64 T2 = (D2 + EW_T2 - 1) / EW_T2, ytiles = D0 * D1 * T2;\n"
+       "  const int tid = threadIdx.x, l3 = (tid % (EW_T3 / EW_V)) * EW_V;\n"
+       "  const i64 TX = (D3 + EW_T3 - 1) / EW_T3, ntiles = ytiles * TX;\n"
        "  for (i64 t = blockIdx.x + (i64)gridDim.x * blockIdx.y; t < ntiles; t += (i64)gridDim.x * gridDim.y) {\n"
        "    const i64 g = t / (EW_GROUP * TX), w = t % (EW_GROUP * TX);\n"
        "    const i64 gs = ytiles - g * EW_GROUP < EW_GROUP ? ytiles - g * EW_GROUP : EW_GROUP;\n"
-       "    const i64 y = g * EW_GROUP + w % gs, u = y / T2, c2_0 = (y % T2) * 64, c1 = u % D1, c0 = u / D1;\n"
+       "    const i64 y = g * EW_GROUP + w % gs, u = y / T2, c2_0 = (y % T2) * EW_T2, c1 = u % D1, c0 = u / D1;\n"
        "    {\n"
-       "      const i64 c3_0 = (w / gs) * 64;\n";
+       "      const i64 c3_0 = (w / gs) * EW_T3;\n";
   for (int k = 0; k < n_inputs; ++k) {
-    if (in_kind[k] == 'v') {
-      // VS elements of axis 2 per thread, 64/VS threads per tile row, 16/VS rows per thread
+    if (in_kind[k] == 'v' || in_kind[k] == 'V') {
+      // VS elements of axis 2 per thread, T2/VS threads per tile row, 16/VS tile rows per thread
       const int vs = (in_dt[k] == IHIP_DT_F32 || in_dt[k] == IHIP_DT_I32) ? 4 : 8;
       s += fmt("      float sv%d[16 / %d][%d];\n"
                "      {\n"
                "        const void* p = a.in_ptr[%d];\n"
                "        const i64 base = c0 * a.in_stride[%d][0] + c1 * a.in_stride[%d][1], s3 = a.in_stride[%d][3];\n"
-               "        const i64 g2 = c2_0 + (tid %% (64 / %d)) * %d;\n"
+               "        const i64 g2 = c2_0 + (tid %% (EW_T2 / %d)) * %d;\n"
                "#pragma unroll\n"
                "        for (int i = 0; i < 16 / %d; ++i) {\n"
-               "          const i64 g3 = c3_0 + i * 4 * %d + tid / (64 / %d);\n"
-               "          ld%d<%d>(p, g2 < D2 && g3 < D3 ? base + g2 + g3 * s3 : base, sv%d[i]);\n"
+               "          const i64 g3 = c3_0 + i * (256 * %d / EW_T2) + tid / (EW_T2 / %d);\n"
+               "          ld%d%s<%d>(p, g2 < D2 && g3 < D3 ? base + g2 + g3 * s3 : base, sv%d[i]);\n"
                "        }\n"
                "      }\n",
-               k, vs, vs, k, k, k, k, vs, vs, vs, vs, vs, vs, in_dt[k], k);
+               k, vs, vs, k, k, k, k, vs, vs, vs, vs, vs, vs, in_kind[k] == 'V' ? "c" : "", in_dt[k], k);
     } else if (in_kind[k] == 't') {
       s += fmt("      float sv%d[16];\n"
                "      {\n"
                "        const void* p = a.in_ptr[%d];\n"
                "        const i64 base = c0 * a.in_stride[%d][0] + c1 * a.in_stride[%d][1], s3 = a.in_stride[%d][3];\n"
-               "        const i64 g2 = c2_0 + (tid & 63);\n"
+               "        const i64 g2 = c2_0 + tid %% EW_T2;\n"
                "#pragma unroll\n"
                "        for (int i = 0; i < 16; ++i) {\n"
-               "          const i64 g3 = c3_0 + (tid >> 6) + 4 * i;\n"
+               "          const i64 g3 = c3_0 + tid / EW_T2 + 256 / EW_T2 * i;\n"
                "          sv%d[i] = ld1<%d>(p, g2 < D2 && g3 < D3 ? base + g2 + g3 * s3 : base);\n"
                "        }\n"
                "      }\n",
@@ -769,7 +780,7 @@ std::string ew_jit_source(const ihip_ew_instr* code, int n_code, int n_inputs, c
   if (loaded) {
     s += "#pragma unroll\n"
          "      for (int pass = 0; pass < 16 / EW_V; ++pass) {\n"
-         "        const i64 c2 = c2_0 + pass * 4 * EW_V + tid / (64 / EW_V), c2c = c2 < D2 ? c2 : D2 - 1;\n";
+         "        const i64 c2 = c2_0 + pass * (256 * EW_V / EW_T3) + tid / (EW_T3 / EW_V), c2c = c2 < D2 ? c2 : D2 - 1;\n";
     for (int k = 0; k < n_inputs; ++k)
       if ((loaded >> k) & 1u)
         s += fmt("        ldk<%d, '%c'>(a.in_ptr[%d], c0 * a.in_stride[%d][0] + c1 * a.in_stride[%d][1] + c2c * "
@@ -780,24 +791,25 @@ std::string ew_jit_source(const ihip_ew_instr* code, int n_code, int n_inputs, c
   s += "      __syncthreads();  // the previous tile is consumed\n";
   int slot = 0;
   for (int k = 0; k < n_inputs; ++k) {
-    if (in_kind[k] == 'v') {
+    if (in_kind[k] == 'v' || in_kind[k] == 'V') {
       const int vs = (in_dt[k] == IHIP_DT_F32 || in_dt[k] == IHIP_DT_I32) ? 4 : 8;
       s += fmt("#pragma unroll\n"
                "      for (int i = 0; i < 16 / %d; ++i)\n"
                "        for (int e = 0; e < %d; ++e)\n"
-               "          tile[%d][i * 4 * %d + tid / (64 / %d)][(tid %% (64 / %d)) * %d + e] = sv%d[i][e];\n",
+               "          tile[%d][i * (256 * %d / EW_T2) + tid / (EW_T2 / %d)][(tid %% (EW_T2 / %d)) * %d + e] = sv%d[i][e];\n",
                vs, vs, slot, vs, vs, vs, vs, k);
       ++slot;
     } else if (in_kind[k] == 't') {
       s += fmt("#pragma unroll\n"
-               "      for (int i = 0; i < 16; ++i) tile[%d][(tid >> 6) + 4 * i][tid & 63] = sv%d[i];\n", slot, k);
+               "      for (int i = 0; i < 16; ++i) tile[%d][tid / EW_T2 + 256 / EW_T2 * i][tid %% EW_T2] = sv%d[i];\n", slot,
+               k);
       ++slot;
     }
   }
   s += "      __syncthreads();\n"
        "#pragma unroll\n"
        "      for (int pass = 0; pass < 16 / EW_V; ++pass) {\n"
-       "        const int l2 = pass * 4 * EW_V + tid / (64 / EW_V);\n"
+       "        const int l2 = pass * (256 * EW_V / EW_T3) + tid / (EW_T3 / EW_V);\n"
        "        const i64 c2 = c2_0 + l2, row = (c0 * D1 + c1) * D2 + c2;\n"
        "        if (c2 < D2 && c3 < D3) {\n"
        "          float r[EW_NREG][EW_V];\n";
@@ -904,10 +916,11 @@ struct JitForm {
   char in_kind[IHIP_EW_NATIVE_MAX_INPUTS + 1] = {}, out_kind[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = {};
   uint32_t rowinv = 0;
   bool flat = false;
+  bool wide = false;  // tiled form: 128 x 32 tiles instead of 64 x 64
 
   std::string source() const {
     return flat ? ew_jit_source_flat(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind)
-                : ew_jit_source(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind, out_kind, rowinv);
+                : ew_jit_source(code, n_code, n_inputs, in_dt, n_outputs, out_dt, in_kind, out_kind, rowinv, wide);
   }
 
   // The same, as the cache's key: a launch looks its code up by this and writes no source (that
@@ -916,7 +929,7 @@ struct JitForm {
     std::string k;
     k.reserve(16 + 9 * n_code + 2 * (n_inputs + n_outputs));
     const auto put32 = [&](uint32_t v) { k.append(reinterpret_cast<const char*>(&v), sizeof v); };
-    k.push_back(flat ? 'f' : 'r');
+    k.push_back(flat ? 'f' : wide ? 'w' : 'r');
     put32(static_cast<uint32_t>(n_code));
     put32(rowinv);
     for (int pc = 0; pc < n_code; ++pc) {
@@ -1057,13 +1070,34 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     return shape[2] % vs == 0 && st[3] % vs == 0 && (st[0] % vs == 0 || shape[0] == 1) &&
            (st[1] % vs == 0 || shape[1] == 1) && reinterpret_cast<uintptr_t>(inputs[k].ptr) % 16 == 0;
   };
+  // Tile of the tiled form: 128 x 32 where every operand is 4 bytes wide and the staged ones are
+  // read in vectors: both sides of a tile are whole 128-byte lines, and the reads 512 bytes
+  // ([8192, 8192] 105.0 -> 97.4 us).  64 x 64 where 32 columns of a 16-bit operand would be half a
+  // line, for element-wise staging ([8191, 4099] 90.2 us, in 128 x 32 tiles 95.1), for axis 2 of at most
+  // 64, and where 128 x 32 takes more tiles.
+  // Staged inputs of 32 bits: ordinary loads ('V') where they and the outputs fit the 256 MB memory-side
+  // cache together, so that what an earlier kernel left there is found (probe, x kept between
+  // passes: [2048, 15360] 46.0 -> 31.0 us, [8192, 1024] 10.3 -> 6.8; over four sets of buffers 47.8 -> 48.7
+  // and 13.2 -> 9.4); non-temporal ('v') above ([8192, 8192] 91.6 us, ordinary 95.7).
+  bool four = true;
+  for (int k = 0; k < n_inputs; ++k) four &= esize(in_dt[k]) == 4 && (!((tile_mask >> k) & 1u) || stage_vec(k));
+  for (int k = 0; k < n_outputs; ++k) four &= esize(out_dt[k]) == 4;
+  f.wide = tile_mask != 0 && four && shape[2] > 64 &&
+           ((shape[2] + 127) / 128) * ((shape[3] + 31) / 32) <= ((shape[2] + 63) / 64) * ((shape[3] + 63) / 64);
+  int64_t tiled_bytes = 0;
+  for (int k = 0; k < n_inputs; ++k) tiled_bytes += ((tile_mask >> k) & 1u) ? esize(in_dt[k]) : 0;
+  for (int k = 0; k < n_outputs; ++k) tiled_bytes += esize(out_dt[k]);
+  const bool cached = tiled_bytes * a.rows * shape[3] <= int64_t(256) * 1000 * 1000;
+  const auto stage_kind = [&](int k) {
+    return !stage_vec(k) ? 't' : esize(in_dt[k]) == 4 && cached ? 'V' : 'v';
+  };
   char(&in_kind)[IHIP_EW_NATIVE_MAX_INPUTS + 1] = f.in_kind;
   char(&out_kind)[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = f.out_kind;
   for (int k = 0; k < n_inputs; ++k) {
     a.in_ptr[k] = inputs[k].ptr;
     for (int d = 0; d < 4; ++d) a.in_stride[k][d] = inputs[k].stride[d];
     const int64_t* st = inputs[k].stride;
-    in_kind[k] = ((tile_mask >> k) & 1u)                          ? (stage_vec(k) ? 'v' : 't')
+    in_kind[k] = ((tile_mask >> k) & 1u)                          ? stage_kind(k)
                  : (V == 8 && vec_ok(inputs[k].ptr, st, in_dt[k], 8)) ? '8'
                  : vec_ok(inputs[k].ptr, st, in_dt[k], 4)               ? '4'
                  : st[3] == 0                                           ? 'b'
@@ -1090,7 +1124,7 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     if (plan_flat(code, n_code, inputs, n_inputs, shape, vectors, V, pl)) return true;
   }
   f.rowinv = rowinv;
-  if (tile_mask != 0) {  // one workgroup per 64 x 64 tile (linear id; grid-strided beyond the grid limits)
+  if (tile_mask != 0) {  // one workgroup per 64 x 64 tile, at most one per 128 x 32 (linear id; grid-strided beyond the grid limits)
     const int64_t tx = (shape[3] + 63) / 64, ty = shape[0] * shape[1] * ((shape[2] + 63) / 64);
     pl.gx = static_cast<unsigned>(tx < 65535 ? tx : 65535);
     pl.gy = static_cast<unsigned>(ty < 65535 ? ty : 65535);

@@ -1054,7 +1054,8 @@ def _ew_launch(prog, dtype_of) -> HipLaunch:
     """The launch ihip_elementwise_program plans (ewjit.hip plan_jit) for dense 16-byte aligned
     outputs: lanes own 8 elements when every operand is 16-bit or narrower, else 4.  Inputs read
     across their unit-stride axis (axis 2 contiguous, axis 3 strided; up to 4) select the
-    LDS-tiled form: one workgroup per 64 x 64 tile, a 64 x 65 f32 tile each.  Otherwise up to
+    LDS-tiled form: one workgroup per 64 x 64 tile, a 64 x 65 f32 tile each (or as many for
+    128 x 32 tiles, 32 x 130 f32 each).  Otherwise up to
     16384 256-lane workgroups stride over groups of U rows and over vectors, or (_ew_flat_workgroups)
     over the whole space as one run of elements."""
     sh = [1] * (4 - len(prog.shape)) + [int(d) for d in prog.shape]
