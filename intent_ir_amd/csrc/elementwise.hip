@@ -116,8 +116,9 @@ __global__ __launch_bounds__(256) void bias_gelu_axpy_bf16_vec(const u32x4* __re
 
 // Rows off 16-byte alignment (N % 8 != 0, or unaligned bases): a lane takes 8 consecutive elements
 // of the whole tensor, kRuns such runs per trip, whatever row they start in, with 16-byte accesses
-// at any 2-byte boundary.  The last run starts 8 before the end and repeats elements of the one
-// before it (the same values are stored twice).  A run's 8 bias values are those from its column
+// at any 2-byte boundary.  The last run starts 8 before the end; of the elements that it shares with
+// the one before it (the first `dup`) nothing is stored, so that y may be x: that run may have stored
+// them before this one reads them.  A run's 8 bias values are those from its column
 // to the row's end, then from column 0: two 16-byte words (one of them the same for every run)
 // shifted against each other.  Against an element per thread, us: [32768, 4099] 229.2 -> 88.8 (6.05
 // TB/s), [7744, 2397] 42.5 -> 14.7, [1000000, 23] 49.5 -> 19.0.  8 <= N, total < 2^31 - 2^13; magic, shift: floor(e / N) as
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(256) void bias_gelu_axpy_bf16_flat(const uint16_t* 
                                                                 uint16_t* __restrict__ y, uint32_t total, uint32_t N,
                                                                 float a, uint32_t magic, uint32_t shift) {
   constexpr int kRuns = 4;
-  const uint32_t nrun = (total + 7) / 8;
+  const uint32_t nrun = (total + 7) / 8, dup = nrun * 8 - total;
   const u32x4 b0 = *reinterpret_cast<const u32x4_b2*>(bias);
   for (uint32_t t0 = blockIdx.x * (256 * kRuns); t0 < nrun; t0 += gridDim.x * (256 * kRuns)) {
     uint32_t e[kRuns];
@@ -160,7 +161,14 @@ __global__ __launch_bounds__(256) void bias_gelu_axpy_bf16_flat(const uint16_t* 
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         o[j] = bf16x2_apply<kFolded>(v[u][j], __uint_as_float(w[u][j] << 16), __uint_as_float(w[u][j] & 0xffff0000u), a);
-      if (t0 + u * 256 + threadIdx.x < nrun) __builtin_nontemporal_store(o, reinterpret_cast<u32x4_b2*>(y + e[u]));
+      const uint32_t run = t0 + u * 256 + threadIdx.x;
+      if (run < nrun - (dup > 0)) {
+        __builtin_nontemporal_store(o, reinterpret_cast<u32x4_b2*>(y + e[u]));
+      } else if (run < nrun) {
+#pragma unroll
+        for (uint32_t j = 1; j < 8; ++j)
+          if (j >= dup) y[e[u] + j] = static_cast<uint16_t>(o[j >> 1] >> (16 * (j & 1)));
+      }
     }
   }
 }

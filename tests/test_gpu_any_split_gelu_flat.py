@@ -100,3 +100,22 @@ def test_gelu_rows_at_any_2_byte_boundary(hip, M, N, ox, ob, oy, alpha):
     got = bf16_bits_to_f32(h[oy:oy + M * N].reshape(M, N)).astype(np.float64)
     assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 2.0 ** -19 * (np.abs(z) + np.abs(xf))).all()
     assert (h[:oy] == 0x1234).all() and (h[oy + M * N:] == 0x1234).all(), "written outside y"
+
+
+@pytest.mark.parametrize("M,N", [(1, 9), (1, 513), (3, 171), (1, 2049), (1, 8193), (7, 1171), (5, 1639), (683, 771)])
+def test_gelu_in_place(hip, M, N):
+    """y may be x: the runs at the end, which share elements across waves and workgroups, included."""
+    import torch
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M * N)
+    x = torch.randn(M, N, device="cuda", generator=gen).bfloat16()
+    b = torch.randn(N, device="cuda", generator=gen).bfloat16()
+    y = torch.empty_like(x)
+    print(f"[case] gelu in place M={M} N={N}", flush=True)
+    for out in (y, x):
+        st = hip.ihip_bias_gelu_tanh_axpy_bf16(P(x.data_ptr()), P(b.data_ptr()), P(out.data_ptr()), M, N,
+                                               ctypes.c_float(0.5), _stream(torch))
+        assert st == 0, hip.ihip_last_error().decode()
+    torch.cuda.synchronize()
+    assert torch.equal(x, y)
