@@ -280,6 +280,12 @@ template <int DT> __device__ __forceinline__ void stu(void* p, i64 i, const floa
                                 (u32x4_e4*)((int*)p + i));
   }
 }
+// stu without the first `dup` elements (dup >= 1).
+template <int DT> __device__ __forceinline__ void sttail(void* p, i64 i, u32 dup, const float* v) {
+#pragma unroll
+  for (int j = 1; j < EW_V; ++j)
+    if ((u32)j >= dup) st1<DT>(p, i + j, v[j]);
+}
 // One operand's EW_V elements in the flat form, for the run of elements starting at e = row * D3
 // + col.  Kinds: 'u' one per element (dense), 'b' one value, and, per column (a bias) or per row
 // of D3 elements: 'x' / 'c' when a run stays inside one row (D3 % EW_V == 0), 'w' / 'd' when it may
@@ -606,7 +612,9 @@ static std::string ew_jit_body(const ihip_ew_instr* code, int n_code, const int*
         break;
       case IHIP_EW_STORE:
         if (flat)
-          s += fmt("%sif (live[u]) stu<%d>(a.out_ptr[%d], (i64)e[u], r[%d]);\n", ind, out_dt[in.b], in.b, in.a);
+          s += fmt("%sif (live[u]) stu<%d>(a.out_ptr[%d], (i64)e[u], r[%d]);\n"
+                   "%selse if (last[u]) sttail<%d>(a.out_ptr[%d], (i64)e[u], dup, r[%d]);\n",
+                   ind, out_dt[in.b], in.b, in.a, ind, out_dt[in.b], in.b, in.a);
         else if (preload)
           s += fmt("%sif (live[u]) stk<%d, '%c'>(a.out_ptr[%d], (rb + u) * D3 + c3, valid, r[%d]);\n", ind,
                    out_dt[in.b], out_kind[in.b], in.b, in.a);
@@ -820,8 +828,9 @@ std::string ew_jit_source(const ihip_ew_instr* code, int n_code, int n_inputs, c
 
 // Flat form (plan_flat): every lane takes EW_V consecutive elements of the whole iteration space,
 // EW_U such runs per trip with their loads issued together.  The last run starts EW_V before the
-// end and repeats elements of the one before it (the same values are stored twice), so no run is
-// partial and no load sits behind a branch.
+// end, so no run is partial and no load sits behind a branch; of the elements that it shares with
+// the one before it (the first `dup`) nothing is stored, so that an output may be an input: that run
+// may have stored them before this one reads them.
 std::string ew_jit_source_flat(const ihip_ew_instr* code, int n_code, int n_inputs, const int* in_dt, int n_outputs,
                                const int* out_dt, const char* in_kind) {
   const int V = ew_jit_width(n_inputs, in_dt, n_outputs, out_dt);
@@ -838,18 +847,19 @@ std::string ew_jit_source_flat(const ihip_ew_instr* code, int n_code, int n_inpu
                       ew_jit_rows_per_trip(code, n_code, V, scalars));
   s += kPrelude;
   s += "extern \"C\" __global__ __launch_bounds__(256) void ihip_ew_jit(const EwJitArgs a) {\n"
-       "  const u32 d3 = (u32)a.shape[3], nrun = (a.total + EW_V - 1) / EW_V;\n";
+       "  const u32 d3 = (u32)a.shape[3], nrun = (a.total + EW_V - 1) / EW_V, dup = nrun * EW_V - a.total;\n";
   for (int pc = 0; pc < n_code; ++pc)
     if (code[pc].op == IHIP_EW_LOAD && ((scalars >> code[pc].a) & 1u))
       s += fmt("  float L%d[1][EW_V];\n  ldf<%d, 'b'>(a.in_ptr[%d], 0, 0, 0, d3, L%d[0]);\n", pc, in_dt[code[pc].a],
                (int)code[pc].a, pc);
   s += "  for (u32 t0 = blockIdx.x * (256 * EW_U); t0 < nrun; t0 += gridDim.x * (256 * EW_U)) {\n"
        "    u32 e[EW_U], row[EW_U], col[EW_U];\n"
-       "    bool live[EW_U];\n"
+       "    bool live[EW_U], last[EW_U];\n"
        "#pragma unroll\n"
        "    for (int u = 0; u < EW_U; ++u) {\n"
        "      const u32 run = t0 + u * 256 + threadIdx.x;\n"
-       "      live[u] = run < nrun;\n"
+       "      live[u] = run < nrun - (dup > 0);\n"
+       "      last[u] = dup > 0 && run == nrun - 1;\n"
        "      e[u] = run < nrun - 1 ? run * EW_V : a.total - EW_V;\n";
   s += rows ? "      row[u] = (u32)(((unsigned long long)e[u] * a.magic) >> a.shift);\n"
               "      col[u] = e[u] - row[u] * d3;\n"

@@ -88,3 +88,24 @@ def test_flat_form_equals_the_interpreter_kernel(hip, shape, types):
             got[mode] = whole
         for n in "yz":
             assert torch.equal(got[EW_MODE_NATIVE][n], got[EW_MODE_INTERP][n]), f"{n} differs"
+
+
+@pytest.mark.parametrize("dt,V", [("f32", 4), ("bf16", 8), ("i32", 4)])
+@pytest.mark.parametrize("total", [9, 64, 65, 67, 129, 257, 1025])  # in runs of V, and 1 or 3 elements more
+def test_flat_form_in_place(hip, dt, V, total):
+    """An output may be an input: the last run shares elements with one of another wave or workgroup."""
+    import torch
+
+    from intent_ir_amd import launch_lowered, lower_intent_to_hip_kernel
+
+    N = total // 64 * 64 * V + total % 64
+    ir = {"name": "bump", "tensors": {n: {"dtype": dt, "shape": ["M", "N"]} for n in "xyb"},
+          "ops": [{"op": "add", "inputs": ["x", "b"], "output": "y"}], "outputs": ["y"]}
+    k = lower_intent_to_hip_kernel(ir, shape_bindings={"M": 1, "N": N})
+    x = torch.arange(N, device="cuda").remainder(50).to(torch_dtype(dt)).view(1, N)
+    b = torch.ones_like(x)
+    want = x + b
+    print(f"[case] flat in place {dt} N={N}", flush=True)
+    launch_lowered(k, {"x": x, "b": b, "y": x})
+    torch.cuda.synchronize()
+    assert torch.equal(x, want)
