@@ -15,6 +15,7 @@ library or a ROCm device, calls raise ``HipRuntimeError``.
 
 from __future__ import annotations
 
+import copy
 import ctypes
 import threading
 from pathlib import Path
@@ -222,12 +223,13 @@ class _CallPlan:
     bound shapes, the entry point, and the C arguments that are not pointers.  Nothing of a buffer is
     kept, and nothing here is written after it is built, so threads may share it."""
 
-    __slots__ = ("io_spec", "bindings", "bound", "call_args", "kernel_id", "tensors", "fn", "args", "ptr_slots",
+    __slots__ = ("io_spec", "bindings", "bound", "spec", "call_args", "kernel_id", "tensors", "fn", "args", "ptr_slots",
                  "workspaces", "program")
 
     def __init__(self, lowered) -> None:
         self.io_spec, self.bindings = lowered.io_spec, lowered.bindings
         self.bound = dict(lowered.bindings)
+        self.spec = copy.deepcopy(lowered.io_spec["tensors"])
         self.call_args, self.kernel_id = lowered.call_args, lowered.kernel_id
         shapes = tensor_shapes(lowered.io_spec, lowered.bindings)
         self.tensors = tuple((n, spec["dtype"], torch_dtype(spec["dtype"]), shapes[n])
@@ -265,7 +267,7 @@ class _CallPlan:
     def of(self, lowered) -> bool:
         return (self.io_spec is lowered.io_spec and self.call_args is lowered.call_args
                 and self.kernel_id == lowered.kernel_id and self.bindings is lowered.bindings
-                and self.bound == lowered.bindings)
+                and self.bound == lowered.bindings and self.spec == lowered.io_spec["tensors"])
 
 
 def _call_plan(lowered) -> _CallPlan:

@@ -99,3 +99,14 @@ def test_one_kernel_from_several_threads_and_streams(hip):
     for rows in data:
         for x, b, y in rows:
             assert torch.equal(y, x * 2.0 + b)
+
+
+def test_a_changed_io_spec_is_seen(hip):
+    import torch
+
+    k = lower_intent_to_hip_kernel(softmax_inner_ir(), shape_bindings={"M": 5, "N": 96})
+    good = {"input_ptr": torch.randn(5, 96, device="cuda"), "output_ptr": torch.empty(5, 96, device="cuda")}
+    launch_lowered(k, good)
+    k.io_spec["tensors"]["input_ptr"]["dtype"] = "f16"
+    with pytest.raises(HipRuntimeError, match="dtype"):
+        launch_lowered(k, good)
