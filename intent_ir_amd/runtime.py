@@ -317,9 +317,13 @@ def launch_lowered(lowered, buffers: Mapping[str, Any], stream=None) -> None:
         args[i] = ptrs[n]
     keep = []
     for i, nbytes in plan.workspaces:
-        t = torch.empty(max(1, nbytes), dtype=torch.uint8, device="cuda")
-        if stream is not None:  # allocated on the current stream, used on this one
-            t.record_stream(stream)
+        if stream is None:
+            t = torch.empty(max(1, nbytes), dtype=torch.uint8, device="cuda")
+        else:
+            # from that stream's pool: a block of the current stream's may still be in use by work queued
+            # there before it was freed, which the launch would not wait for
+            with torch.cuda.stream(stream):
+                t = torch.empty(max(1, nbytes), dtype=torch.uint8, device="cuda")
         keep.append(t)
         args[i] = t.data_ptr()
     if plan.program is not None:  # operand tables of this call's own
