@@ -1080,27 +1080,35 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     return shape[2] % vs == 0 && st[3] % vs == 0 && (st[0] % vs == 0 || shape[0] == 1) &&
            (st[1] % vs == 0 || shape[1] == 1) && reinterpret_cast<uintptr_t>(inputs[k].ptr) % 16 == 0;
   };
-  // Tile of the tiled form: 128 x 32 where every operand is 4 bytes wide and the staged ones are
-  // read in vectors: both sides of a tile are whole 128-byte lines, and the reads 512 bytes
-  // ([8192, 8192] 105.0 -> 97.4 us).  64 x 64 where 32 columns of a 16-bit operand would be half a
-  // line, for element-wise staging ([8191, 4099] 90.2 us, in 128 x 32 tiles 95.1), for axis 2 of at most
-  // 64, and where 128 x 32 takes more tiles.
-  // Staged inputs of 32 bits: ordinary loads ('V') where they and the outputs fit the 256 MB memory-side
-  // cache together, so that what an earlier kernel left there is found (probe, x kept between
-  // passes: [2048, 15360] 46.0 -> 31.0 us, [8192, 1024] 10.3 -> 6.8; over four sets of buffers 47.8 -> 48.7
-  // and 13.2 -> 9.4); non-temporal ('v') above ([8192, 8192] 91.6 us, ordinary 95.7).
-  bool four = true;
+  // Tile of the tiled form: 64 x 64, or 128 x 32 (staging reads of 512 bytes instead of 256) where
+  // every operand is 4 bytes wide, the staged ones are read in vectors, axis 2 is longer than 64, and
+  // the output lines that a tile writes are its own:
+  //  * rows of at most 32 elements: a tile writes one run of 128 rows, with fewer idle columns too;
+  //  * whole 128-byte lines per tile (rows a multiple of 32, output bases aligned), no more tiles than
+  //    of 64 x 64, and more than 256 MB moved.
+  // us on 64 x 64 -> 128 x 32, over the same buffers and over four sets: [493444, 17] 39.3 -> 22.6, 39.5 ->
+  // 23.7; [524288, 32] 25.9 -> 23.8, 26.8 -> 25.6; [8192, 8192] 103.2 -> 98.1; [699008, 96] 101.7 ->
+  // 90.6; [4096, 8192] 53.3 -> 50.9, 55.0 -> 51.4.  On the other side of the line: rows that are not
+  // whole lines, whose pieces two workgroups share, [8192, 4100] 63.2 -> 86.3, 65.8 -> 87.3, [524288, 33]
+  // 48.3 -> 69.8, 48.8 -> 72.4; up to 256 MB [8192, 1024] 13.6 -> 15.4, 16.1 -> 17.0, [131072, 64] 11.7
+  // -> 16.4, 15.6 -> 16.9.
+  // Vectors of 32-bit staged inputs are read past the caches ('v'), but with ordinary loads ('V') for rows
+  // of at most 32 elements while they and the outputs fit the 256 MB memory-side cache together, where
+  // that gained over the same buffers and over four sets ([493444, 17] 27.0 -> 22.6, 27.4 -> 23.7; [524288, 32] 26.0 -> 23.8,
+  // 27.5 -> 25.6); longer rows lose over rotating buffers ([98304, 256] 38.7 -> 32.4 but 39.4 -> 42.9).
+  bool four = true, lines = shape[3] % 32 == 0;
   for (int k = 0; k < n_inputs; ++k) four &= esize(in_dt[k]) == 4 && (!((tile_mask >> k) & 1u) || stage_vec(k));
-  for (int k = 0; k < n_outputs; ++k) four &= esize(out_dt[k]) == 4;
-  f.wide = tile_mask != 0 && four && shape[2] > 64 &&
-           ((shape[2] + 127) / 128) * ((shape[3] + 31) / 32) <= ((shape[2] + 63) / 64) * ((shape[3] + 63) / 64);
+  for (int k = 0; k < n_outputs; ++k) {
+    four &= esize(out_dt[k]) == 4;
+    lines &= reinterpret_cast<uintptr_t>(outputs[k].ptr) % 128 == 0;
+  }
+  lines &= ((shape[2] + 127) / 128) * (shape[3] / 32) <= ((shape[2] + 63) / 64) * ((shape[3] + 63) / 64);
   int64_t tiled_bytes = 0;
   for (int k = 0; k < n_inputs; ++k) tiled_bytes += ((tile_mask >> k) & 1u) ? esize(in_dt[k]) : 0;
   for (int k = 0; k < n_outputs; ++k) tiled_bytes += esize(out_dt[k]);
   const bool cached = tiled_bytes * a.rows * shape[3] <= int64_t(256) * 1000 * 1000;
-  const auto stage_kind = [&](int k) {
-    return !stage_vec(k) ? 't' : esize(in_dt[k]) == 4 && cached ? 'V' : 'v';
-  };
+  f.wide = tile_mask != 0 && four && shape[2] > 64 && (shape[3] <= 32 || (lines && !cached));
+  const auto stage_kind = [&](int k) { return !stage_vec(k) ? 't' : f.wide && cached ? 'V' : 'v'; };
   char(&in_kind)[IHIP_EW_NATIVE_MAX_INPUTS + 1] = f.in_kind;
   char(&out_kind)[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = f.out_kind;
   for (int k = 0; k < n_inputs; ++k) {
@@ -1134,7 +1142,8 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
     if (plan_flat(code, n_code, inputs, n_inputs, shape, vectors, V, pl)) return true;
   }
   f.rowinv = rowinv;
-  if (tile_mask != 0) {  // one workgroup per 64 x 64 tile, at most one per 128 x 32 (linear id; grid-strided beyond the grid limits)
+  if (tile_mask != 0) {  // one workgroup per 64 x 64 tile, at most one per 128 x 32 (linear id; grid-strided
+                         // beyond the grid limits)
     const int64_t tx = (shape[3] + 63) / 64, ty = shape[0] * shape[1] * ((shape[2] + 63) / 64);
     pl.gx = static_cast<unsigned>(tx < 65535 ? tx : 65535);
     pl.gy = static_cast<unsigned>(ty < 65535 ? ty : 65535);

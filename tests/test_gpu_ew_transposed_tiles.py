@@ -1,8 +1,9 @@
 """Tiles of element-wise programs with inputs read across their unit-stride axis (ewjit.hip
-plan_jit): 128 x 32 where every operand is 4 bytes wide, the staged ones are read in vectors
-and that takes no more tiles, 64 x 64 otherwise, at extents around both tiles, with aligned and unaligned bases.  The program only adds
-and multiplies, each correctly rounded, so the native result must equal the interpreter kernel's
-bit for bit."""
+plan_jit): 128 x 32 where every operand is 4 bytes wide, the staged ones are read in vectors and a
+tile's output lines are its own (rows of at most 32 elements, or whole lines of a large space),
+64 x 64 otherwise, at extents around both tiles, with aligned and unaligned bases.  The program only
+adds and multiplies, each correctly rounded, so the native result must equal the interpreter
+kernel's bit for bit."""
 
 import ctypes
 
@@ -15,9 +16,13 @@ CODE = ((OP["load"], 0, 0, 0, 0, 0.0), (OP["load"], 1, 1, 0, 0, 0.0), (OP["load"
         (OP["mul"], 3, 0, 1, 0, 0.0), (OP["add"], 3, 3, 2, 0, 0.0), (OP["store"], 0, 3, 0, 0, 0.0))
 
 # (batch, axis 2, axis 3), wide in f32
-SHAPES = [((1, 128, 32), True), ((1, 127, 31), False), ((1, 65, 32), False), ((1, 68, 32), True), ((1, 64, 32), False), ((1, 129, 33), False),
-          ((1, 128, 64), True), ((1, 130, 96), False), ((1, 200, 100), True), ((1, 520, 256), False), ((2, 256, 128), True),
-          ((3, 100, 7), True), ((1, 1000, 1), False), ((1, 2, 1000), False), ((1, 1024, 1028), True), ((2, 255, 257), False)]
+SHAPES = [((1, 128, 32), True), ((1, 127, 31), False), ((1, 65, 32), False), ((1, 68, 32), True), ((1, 64, 32), False),
+          ((1, 129, 33), False), ((1, 128, 64), False), ((1, 130, 96), False), ((1, 200, 100), False),
+          ((1, 520, 256), False), ((2, 256, 128), False), ((3, 100, 7), True), ((1, 1000, 1), False), ((1, 2, 1000), False),
+          ((1, 1024, 1028), False), ((2, 255, 257), False), ((1, 1000, 20), True), ((5, 132, 31), True)]
+# the same above 256 MB: whole lines only, and no more tiles of 128 x 32 than of 64 x 64
+LARGE = [((1, 8192, 8192), True), ((1, 8192, 4128), True), ((1, 8192, 4100), False), ((1, 8192, 4112), False),
+         ((1, 8191, 4128), False), ((1, 5800, 5888), False), ((1, 1048576, 33), False), ((1, 1048576, 32), True)]
 TYPES = [("f32", "f32", "f32", "f32"), ("i32", "f32", "f32", "f32"), ("bf16", "f32", "f32", "f32"),
          ("f32", "f32", "f32", "f16"), ("f16", "f16", "f16", "f16")]
 
@@ -27,23 +32,31 @@ def _program(shape):
     return EwProgram(CODE, (("a", (r * c, 0, 1, r)), ("b", (r * c, 0, c, 1)), ("c", (0, 0, 0, 1))), ("y",), (b, 1, r, c))
 
 
-@pytest.mark.parametrize("shape,wide", SHAPES)
+@pytest.mark.parametrize("shape,wide", SHAPES + LARGE)
 def test_tile_extents_follow_types_and_shape(shape, wide):
-    """CPU: which tile a launch compiles, and the staging loads (ordinary up to 256 MB moved)."""
+    """CPU: which tile a launch compiles, and the staging loads (ordinary for short rows up to 256 MB
+    moved)."""
     ptrs = {n: 0x100000 * (i + 1) for i, n in enumerate("abcy")}
     for types in TYPES:
         src = elementwise_source(_program(shape), ptrs, dict(zip("abcy", types)))
-        four = all(t in ("f32", "i32") for t in types)
-        assert ("#define EW_T2 128" in src) == (wide and four)
-        assert "ld4<0>(p" not in src and "ld4<4>(p" not in src
-    types = dict(zip("abcy", TYPES[0]))
-    assert "ld4<0>(p" in elementwise_source(_program((1, 8192, 8192)), ptrs, types)
-    assert "ld4c<0>(p" in elementwise_source(_program((1, 4096, 4096)), ptrs, types)
+        took = wide and all(t in ("f32", "i32") for t in types)
+        assert ("#define EW_T2 128" in src) == took
+        small = 8 * shape[0] * shape[1] * shape[2] <= 256e6
+        assert ("ld4c<0>(p" in src or "ld4c<4>(p" in src) == (took and small)
+
+
+@pytest.mark.parametrize("shape,wide", LARGE)
+def test_wide_tiles_need_output_lines_of_their_own(shape, wide):
+    """CPU: an output off a 128-byte boundary shares its lines between tiles; short rows do not mind."""
+    ptrs = {n: 0x100000 * (i + 1) for i, n in enumerate("abcy")}
+    ptrs["y"] += 16
+    src = elementwise_source(_program(shape), ptrs, dict(zip("abcy", TYPES[0])))
+    assert ("#define EW_T2 128" in src) == (wide and shape[2] <= 32)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("types", TYPES)
-@pytest.mark.parametrize("shape", [s for s, _ in SHAPES] + [(1, 5800, 5888)])  # the last: non-temporal staging
+@pytest.mark.parametrize("shape", [s for s, _ in SHAPES] + [(1, 5800, 5888), (1, 8192, 4128), (1, 1048576, 32)])
 def test_tiled_form_equals_the_interpreter_kernel(hip, shape, types):
     import torch
 
