@@ -252,7 +252,13 @@ int64_t ihip_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int transpose_
  *    f32 sums go to the workspace and a second kernel adds the segments in order, then bias
  *    and activation.  Deterministic; it differs from the unsplit result only by f32
  *    summation order.  Without room for the partials the launch is unsplit, and so is a
- *    launch with tile = 256 (the rule splits 128 x 128 tiles only).
+ *    launch with tile = 256 (the rule splits 128 x 128 tiles only);
+ *  - with tile = 0, a product of few rows (A as [M, K], M <= 128, 16 <= N <= 65536; gemm_direct.hip
+ *    gemm_direct_takes) runs a kernel that streams B once, of any alignment, without copies:
+ *    up to 8 waves take consecutive ranges of K each and add their sums in order, and with room
+ *    for the partials K is cut into up to 16 segments over workgroups as well.  Deterministic; C
+ *    differs from the unsplit tiled kernel's by f32 summation order only, also without a
+ *    workspace.  tile = 128 or 256 and the entries above keep the one chain over K.
  * The workspace must stay untouched until the launch completes on the stream. */
 int ihip_gemm_bf16_bias_relu_ws(const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, int64_t M,
                                 int64_t N, int64_t K, int transpose_a, int transpose_b, int relu, int tile,

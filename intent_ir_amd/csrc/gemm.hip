@@ -4,9 +4,9 @@
 //
 // Entry point of the GEMM family: shapes whose rows all start 16-byte aligned (N % 8 == 0,
 // K % 8 == 0, M % 8 == 0 for a transposed A) with 16-byte aligned operands go to
-// gemm_fast.hip, for any M, N and K; products with one small side to gemm_direct.hip (with the
-// automatic tile); every other shape runs the guarded kernel below, which stages operands through
-// registers:
+// gemm_fast.hip, for any M, N and K; every other shape runs the guarded kernel below, which stages
+// operands through registers (the workspace entry has more paths: packed copies, segments of K and,
+// for products of few rows, gemm_direct.hip):
 //  * workgroup tile TB(M) x TB(N), TB = 256, or 128 for grids of at most 128 tiles of 256x256
 //    (half the CUs; as in gemm_fast.hip), K step 64; 256 threads = 4 waves in a 2x2 grid,
 //    each wave owning a TB/2 x TB/2 sub-tile = (TB/64)^2 blocks of v_mfma_f32_32x32x16_bf16;
@@ -278,8 +278,6 @@ hipError_t launch_gemm_bf16_bias_relu(const uint16_t* A, const uint16_t* B, cons
                                       int64_t N, int64_t K, bool transpose_a, bool transpose_b, int relu, int tile,
                                       hipStream_t s) {
   if (M == 0 || N == 0) return hipSuccess;
-  if (tile == 0 && gemm_direct_takes(M, N, K, transpose_a, transpose_b))
-    return launch_gemm_direct(A, B, bias, C, M, N, K, transpose_b, relu, nullptr, 0, s);
   if (gemm_fast_fits(M, N, K, transpose_a, transpose_b, A, B, C))
     return launch_gemm_fast(A, B, bias, C, M, N, K, transpose_a, transpose_b, relu, tile, s, false);
   const int tb = tile != 0 ? tile : gemm_fast_tile_extent(M, N);
@@ -290,7 +288,9 @@ hipError_t launch_gemm_bf16_bias_relu(const uint16_t* A, const uint16_t* B, cons
 // The same with a workspace (ws, ws_bytes; may be null / 0): operands the tiled kernel cannot
 // read in place are packed into it and the tiled kernel runs on the copies, and a grid of too
 // few tiles is split along K with f32 partials in it (gemm_pack.hip); without a large enough
-// workspace the unsplit tiled kernel or the guarded kernel runs, as above.
+// workspace the unsplit tiled kernel or the guarded kernel runs, as above.  With the automatic tile
+// a product of few rows goes to gemm_direct.hip, whatever the workspace.  That is this entry's only:
+// its waves divide K, and the entries above promise the same bits for every tile and layout.
 hipError_t launch_gemm_bf16_bias_relu_ws(const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C,
                                          int64_t M, int64_t N, int64_t K, bool transpose_a, bool transpose_b, int relu,
                                          int tile, void* ws, int64_t ws_bytes, hipStream_t s) {

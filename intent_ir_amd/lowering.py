@@ -340,13 +340,13 @@ def _match_gemm(c: _Ctx) -> Optional[HipLoweredKernel]:
         launch = HipLaunch(grid, (256, 1, 1), _gemm_fast_lds(t, ta2 if packed else ta))
     else:  # guarded kernel: the same tile choice, a double-buffered {A, Bt} tile pair of 64-k slices
         launch = HipLaunch(grid, (256, 1, 1), 147456 if t == 256 else 73728)
-    if direct:  # one small side: gemm_direct.hip, with or without segments of K in the workspace
+    if direct:  # few rows: gemm_direct.hip, with or without segments of K in the workspace
         launch, S = _gemm_direct_launch(M, N, K, tb)
         ws = _gemm_split_bytes(M, N, S)
-    if ws > 0:
+    if direct or ws > 0:  # (gemm_direct.hip is the workspace entry's, also where it needs none)
         args = [("tensor", a), ("tensor", b), ("tensor", env["bias"][1]) if has_bias else ("null", None),
                 ("tensor", oname), ("i64", M), ("i64", N), ("i64", K), ("i32", int(ta)), ("i32", int(tb)),
-                ("i32", int(relu)), ("i32", tile), ("workspace", ws)]
+                ("i32", int(relu)), ("i32", tile), *([("workspace", ws)] if ws > 0 else [("null", None), ("i64", 0)])]
         return HipLoweredKernel(c.fn.name, "ihip_gemm_bf16_bias_relu_ws", c.io(names), launch, [oname], dict(c.b),
                                 tuple(args))
     kid = ("ihip_gemm_bf16_bias_relu_ex" if tile else "ihip_gemm_bf16_bias_relu_t" if (ta or tb)

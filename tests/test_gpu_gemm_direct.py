@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from intent_ir_amd.dtypes import f32_to_bf16_bits
+from intent_ir_amd.lowering import _gemm_split_bytes as gemm_split_bytes
 from intent_ir_amd.lowering import gemm_direct_plan, gemm_direct_takes, gemm_workspace_bytes
 
 P = ctypes.c_void_p
@@ -101,3 +102,59 @@ def test_direct_product_keeps_nan_and_inf_to_their_rows_and_columns(hip, tb):
     finite[:, N - 1] = finite[:, 5] = False
     np.testing.assert_array_equal(np.isfinite(f), finite)
     assert np.isnan(f[M - 1]).all() and np.isinf(f[:M - 1, 5]).all()
+
+
+def test_lowered_few_row_products_call_the_workspace_entry():
+    """CPU: the entries without a workspace sum K in one chain, so the few-row kernel is the workspace
+    entry's, with or without segments."""
+    from intent_ir_amd import lower_intent_to_hip_kernel
+    from intent_ir_amd.configs import matmul_bias_relu2d_ir
+
+    for M, N, K, S in ((32, 32000, 4096, 1), (16, 1024, 8192, 16)):
+        assert gemm_direct_takes(M, N, K, False, False) and gemm_direct_plan(M, N, K, False)[2] == S
+        k = lower_intent_to_hip_kernel(matmul_bias_relu2d_ir(), shape_bindings={"M": M, "N": N, "K": K})
+        assert k.kernel_id == "ihip_gemm_bf16_bias_relu_ws"
+        assert k.call_args[-2:] == ((("null", None), ("i64", 0)) if S == 1 else
+                                    (("i32", 0), ("workspace", gemm_split_bytes(M, N, S))))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(16, 1024, 8192), (1, 264, 1000), (33, 520, 1003), (128, 513, 4096)])
+def test_entries_without_a_workspace_give_the_same_bits_for_every_tile_and_layout(hip, M, N, K):
+    """Also on shapes of the few-row kernel: one chain over K.  That kernel's result (the workspace
+    entry, automatic tile) differs by the order of its f32 sums only: the two C are within their
+    bf16 roundings (2^-8 of the value each) and their sums' bounds (K 2^-24 sum |a b| each)."""
+    import torch
+
+    assert gemm_direct_takes(M, N, K, False, False)
+    rng = np.random.default_rng(M + N + K)
+    Af, Bf = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((K, N)).astype(np.float32)
+    bias = torch.from_numpy(rng.standard_normal(N).astype(np.float32)).cuda()
+    stream = P(torch.cuda.current_stream().cuda_stream)
+
+    def dev(x):
+        return torch.from_numpy(f32_to_bf16_bits(np.ascontiguousarray(x)).view(np.int16)).cuda().view(torch.bfloat16)
+
+    op = {("A", False): dev(Af), ("A", True): dev(Af.T), ("B", False): dev(Bf), ("B", True): dev(Bf.T)}
+
+    def run(name, ta, tb, *tail):
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        flags = () if name.endswith("relu") else (int(ta), int(tb))
+        st = getattr(hip, name)(P(op["A", ta].data_ptr()), P(op["B", tb].data_ptr()), P(bias.data_ptr()), P(c.data_ptr()),
+                                M, N, K, *flags, 0, *tail, stream)
+        assert st == 0, hip.ihip_last_error().decode()
+        torch.cuda.synchronize()
+        return c
+
+    print(f"[case] entries without a workspace {M}x{N}x{K}", flush=True)
+    want = run("ihip_gemm_bf16_bias_relu", False, False)
+    for ta in (False, True):
+        for tb in (False, True):
+            assert torch.equal(run("ihip_gemm_bf16_bias_relu_t", ta, tb), want), (ta, tb)
+            for tile in (0, 128, 256):
+                assert torch.equal(run("ihip_gemm_bf16_bias_relu_ex", ta, tb, tile), want), (ta, tb, tile)
+    mag = op["A", False].double().abs() @ op["B", False].double().abs()
+    for tb in (False, True):
+        got = run("ihip_gemm_bf16_bias_relu_ws", False, tb, 0, P(None), 0)
+        err = (got.double() - want.double()).abs()
+        assert (err <= want.double().abs() * 2.0 ** -7 + 2 * K * 2.0 ** -24 * mag).all()
