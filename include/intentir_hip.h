@@ -236,7 +236,9 @@ int ihip_gemm_bf16_bias_relu_ex(const uint16_t* A, const uint16_t* B, const floa
  *    S > 1 segments: only grids of 128 x 128 tiles (the automatic choice when at most 128
  *    tiles of 256 x 256 would be busy) are split, into the S (segments of whole 64-k steps, at
  *    least 512 k each, at most 512 workgroups) of least estimated time on K8 = K rounded up
- *    to 8 (gemm_pack.hip split_plan).
+ *    to 8 (gemm_pack.hip split_plan);
+ * or, where they are more, the partials of a product of few rows with tile = 0 (segments x M x
+ * (N rounded up to 4) floats), which uses nothing else.
  * Same shapes and layouts as the entries above (the reference allocates nothing for matmul:
  * its kernels take any shape in place, intentir_to_cuda.py:537-985). */
 int64_t ihip_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int transpose_a, int transpose_b);

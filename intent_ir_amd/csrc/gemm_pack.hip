@@ -205,16 +205,18 @@ hipError_t pack(const uint16_t* src, uint16_t* dst, int64_t R, int64_t K, bool k
 
 }  // namespace
 
-// Workspace bytes for this shape: the partials of gemm_direct.hip's segments where it is taken,
-// else the packed copies it needs, then the split-K partials
-// (0: neither; operands whose only problem is a 2-byte aligned base are packed too when the
-// workspace passed at launch is large enough for them).
+// Workspace bytes for this shape: the packed copies it needs, then the split-K partials (operands
+// whose only problem is a 2-byte aligned base are packed too when the workspace passed at launch is
+// large enough for them), or the partials of gemm_direct.hip's segments where that kernel takes the
+// shape and they are more.  Both, because a launch with tile = 128 or 256 does not go there.
 int64_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, bool ta, bool tb) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  if (gemm_direct_takes(M, N, K, ta, tb)) return split_bytes(M, N, gemm_direct_segments(M, N, K, tb));
   const int64_t K8 = round8(K);
-  return (shape_packs_a(M, K, ta) ? align_up(M * K8 * 2) : 0) + (shape_packs_b(N, K, tb) ? align_up(N * K8 * 2) : 0) +
-         split_bytes(M, N, split_plan(M, N, K8, 0, 0).S);
+  const int64_t tiled = (shape_packs_a(M, K, ta) ? align_up(M * K8 * 2) : 0) +
+                        (shape_packs_b(N, K, tb) ? align_up(N * K8 * 2) : 0) +
+                        split_bytes(M, N, split_plan(M, N, K8, 0, 0).S);
+  const int64_t few = gemm_direct_takes(M, N, K, ta, tb) ? split_bytes(M, N, gemm_direct_segments(M, N, K, tb)) : 0;
+  return tiled > few ? tiled : few;
 }
 
 // Workspace bytes of a split into `splits` segments (0: by the split rule).

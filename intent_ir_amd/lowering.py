@@ -547,13 +547,13 @@ def gemm_pack_bytes(M: int, N: int, K: int, ta: bool, tb: bool) -> int:
 
 def gemm_workspace_bytes(M: int, N: int, K: int, ta: bool, tb: bool) -> int:
     """Workspace bytes of ihip_gemm_bf16_bias_relu_ws (gemm_pack.hip gemm_workspace_bytes): the
-    packed copies, then the split-K partials of the split rule on K rounded up to 8; 0 when
-    neither is needed."""
+    packed copies, then the split-K partials of the split rule on K rounded up to 8 (for any tile),
+    or the few-row kernel's partials where they are more; 0 when none is needed."""
     if M <= 0 or N <= 0 or K <= 0:
         return 0
-    if gemm_direct_takes(M, N, K, ta, tb):
-        return _gemm_split_bytes(M, N, gemm_direct_plan(M, N, K, tb)[2])
-    return gemm_pack_bytes(M, N, K, ta, tb) + _gemm_split_bytes(M, N, gemm_split_plan(M, N, _cdiv(K, 8) * 8)[0])
+    few = _gemm_split_bytes(M, N, gemm_direct_plan(M, N, K, tb)[2]) if gemm_direct_takes(M, N, K, ta, tb) else 0
+    return max(few, gemm_pack_bytes(M, N, K, ta, tb)
+               + _gemm_split_bytes(M, N, gemm_split_plan(M, N, _cdiv(K, 8) * 8)[0]))
 
 
 def _match_reduce_any(c: _Ctx) -> Optional[HipLoweredKernel]:

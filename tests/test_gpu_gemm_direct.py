@@ -10,7 +10,8 @@ import pytest
 
 from intent_ir_amd.dtypes import f32_to_bf16_bits
 from intent_ir_amd.lowering import _gemm_split_bytes as gemm_split_bytes
-from intent_ir_amd.lowering import gemm_direct_plan, gemm_direct_takes, gemm_workspace_bytes
+from intent_ir_amd.lowering import (gemm_direct_plan, gemm_direct_takes, gemm_pack_bytes, gemm_split_plan,
+                                    gemm_workspace_bytes)
 
 P = ctypes.c_void_p
 GUARD = 64
@@ -30,6 +31,19 @@ def test_lowering_follows_the_library(M, N, K, tb):
     from intent_ir_amd.runtime import load_library
 
     assert load_library().ihip_gemm_workspace_size(M, N, K, 0, int(tb)) == gemm_workspace_bytes(M, N, K, False, tb)
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("tb", [False, True])
+def test_workspace_size_holds_what_a_fixed_tile_needs(M, N, K, tb):
+    """CPU: the size has no tile argument, so it also covers tile = 128 or 256: the packed copies of
+    ragged operands and the tiled kernel's partials, beside the few-row kernel's."""
+    from intent_ir_amd.runtime import load_library
+
+    size = load_library().ihip_gemm_workspace_size(M, N, K, 0, int(tb))
+    tiled = gemm_pack_bytes(M, N, K, False, tb) + gemm_split_bytes(M, N, gemm_split_plan(M, N, -(-K // 8) * 8)[0])
+    few = gemm_split_bytes(M, N, gemm_direct_plan(M, N, K, tb)[2]) if gemm_direct_takes(M, N, K, False, tb) else 0
+    assert size == max(tiled, few)
 
 
 def _run(hip, torch, A, B, bias, M, N, K, tb, relu, offs, ws_bytes):
@@ -68,8 +82,8 @@ def test_direct_product_is_exact_on_integers(hip, M, N, K, tb):
     bias = rng.integers(-8, 9, size=N).astype(np.float32)
     full = (torch.from_numpy(Af).cuda().double() @ torch.from_numpy(Bf).cuda().double()).cpu().numpy()
     A, B = f32_to_bf16_bits(Af), f32_to_bf16_bits(np.ascontiguousarray(Bf.T) if tb else Bf)
-    need = gemm_workspace_bytes(M, N, K, False, tb)
     S = gemm_direct_plan(M, N, K, tb)[2]
+    need = gemm_split_bytes(M, N, S)
     assert (need > 0) == (S > 1)
     for relu, bs, offs in ((True, bias, (0, 0, 0)), (False, None, (1, 3, 1)), (True, bias, (0, 1, 5))):
         ref = full if bs is None else full + bs
