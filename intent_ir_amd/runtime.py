@@ -271,12 +271,16 @@ class _CallPlan:
 
 
 def _call_plan(lowered) -> _CallPlan:
-    """The kernel's plan: kept in the lowered object itself (and rebuilt if its parts were replaced)."""
-    plan = lowered.__dict__.get("_call_plan")
+    """The kernel's plan: kept in the lowered object itself (and rebuilt if its parts were replaced), or
+    built for the call where the object has no attributes of its own to keep it in."""
+    own = getattr(lowered, "__dict__", None)
+    own = own if type(own) is dict else None  # slots, a named tuple, a class
+    plan = own.get("_call_plan") if own is not None else None
     if plan is None or not plan.of(lowered):
         _torch()  # no device: that error first
         plan = _CallPlan(lowered)
-        lowered.__dict__["_call_plan"] = plan
+        if own is not None:
+            own["_call_plan"] = plan
     return plan
 
 
