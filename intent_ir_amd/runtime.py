@@ -224,7 +224,7 @@ class _CallPlan:
     kept, and nothing here is written after it is built, so threads may share it."""
 
     __slots__ = ("io_spec", "bindings", "bound", "spec", "call_args", "kernel_id", "tensors", "fn", "args", "ptr_slots",
-                 "workspaces", "program")
+                 "undescribed", "workspaces", "program")
 
     def __init__(self, lowered) -> None:
         self.io_spec, self.bindings = lowered.io_spec, lowered.bindings
@@ -263,6 +263,7 @@ class _CallPlan:
                 raise HipRuntimeError(f"unknown call argument kind {kind}")
         args.append(None)  # the stream
         self.args, self.ptr_slots, self.workspaces = args, tuple(slots), tuple(workspaces)
+        self.undescribed = tuple({n for _, n in slots} - set(shapes))  # tensors that io_spec does not name
 
     def of(self, lowered) -> bool:
         return (self.io_spec is lowered.io_spec and self.call_args is lowered.call_args
@@ -307,15 +308,14 @@ def launch_lowered(lowered, buffers: Mapping[str, Any], stream=None) -> None:
     Tensor = torch.Tensor
     ptrs = {}
     for n, dt, tdt, shape in plan.tensors:
-        t = buffers.get(n)
-        if (isinstance(t, Tensor) and t.is_cuda and t.dtype is tdt and t.shape == shape and t.is_contiguous()):
-            ptrs[n] = t.data_ptr()
-            continue
-        _torch()
         if n not in buffers:
             raise HipRuntimeError(f"missing buffer for {n}")
-        _check_buffer(n, t, dt, shape)  # raises, unless t is the bound shape in another arrangement of its axes
+        t = buffers[n]
+        if not (isinstance(t, Tensor) and t.is_cuda and t.dtype is tdt and t.shape == shape and t.is_contiguous()):
+            _check_buffer(n, t, dt, shape)  # raises, unless t is the bound shape in another arrangement of its axes
         ptrs[n] = t.data_ptr()
+    for n in plan.undescribed:
+        ptrs[n] = buffers[n].data_ptr()
     args = plan.args.copy()
     for i, n in plan.ptr_slots:
         args[i] = ptrs[n]

@@ -57,3 +57,37 @@ def test_any_object_with_the_fields_is_launched(calls, kind):
         launch_lowered(lowered, b)
     assert len(calls) == 2 and calls[0] == calls[1]
     assert calls[0][:2] == (b["input_ptr"].data_ptr(), b["output_ptr"].data_ptr()) and calls[0][-1] == 5
+
+
+class _Named:
+    """Buffers with the two operations that a launch needs."""
+
+    def __init__(self, d):
+        self.d = d
+
+    def __contains__(self, n):
+        return n in self.d
+
+    def __getitem__(self, n):
+        return self.d[n]
+
+
+def test_buffers_need_only_membership_and_lookup(calls):
+    k, b = _kernel(), _buffers()
+    launch_lowered(k, _Named(b))
+    assert calls[0][:2] == (b["input_ptr"].data_ptr(), b["output_ptr"].data_ptr())
+    del b["output_ptr"]
+    with pytest.raises(runtime.HipRuntimeError, match="missing buffer for output_ptr"):
+        launch_lowered(k, _Named(b))
+
+
+def test_an_argument_outside_the_io_spec_is_passed(calls):
+    """A call plan may name a tensor that io_spec does not describe: it is passed unchecked."""
+    import torch
+
+    k, b = _kernel(), _buffers()
+    b["extra"] = torch.zeros(3)
+    lowered = SimpleNamespace(io_spec=k.io_spec, bindings=k.bindings, kernel_id=k.kernel_id,
+                              call_args=(*k.call_args, ("tensor", "extra")))
+    launch_lowered(lowered, b)
+    assert calls[0][-2] == b["extra"].data_ptr()
