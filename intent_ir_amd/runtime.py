@@ -223,14 +223,17 @@ class _CallPlan:
     bound shapes, the entry point, and the C arguments that are not pointers.  Nothing of a buffer is
     kept, and nothing here is written after it is built, so threads may share it."""
 
-    __slots__ = ("io_spec", "bindings", "bound", "spec", "call_args", "kernel_id", "tensors", "fn", "args", "ptr_slots",
-                 "undescribed", "workspaces", "program")
+    __slots__ = ("io_spec", "bindings", "bound", "spec", "call_args", "fixed", "seen", "kernel_id", "tensors", "fn",
+                 "args", "ptr_slots", "undescribed", "workspaces", "program")
 
     def __init__(self, lowered) -> None:
         self.io_spec, self.bindings = lowered.io_spec, lowered.bindings
         self.bound = dict(lowered.bindings)
         self.spec = copy.deepcopy(lowered.io_spec["tensors"])
         self.call_args, self.kernel_id = lowered.call_args, lowered.kernel_id
+        # pairs that cannot change under the plan are recognised by the tuple that holds them
+        self.fixed = type(self.call_args) is tuple and all(type(a) is tuple for a in self.call_args)
+        self.seen = tuple((kind, v) for kind, v in self.call_args)
         shapes = tensor_shapes(lowered.io_spec, lowered.bindings)
         self.tensors = tuple((n, spec["dtype"], torch_dtype(spec["dtype"]), shapes[n])
                              for n, spec in lowered.io_spec["tensors"].items())
@@ -266,7 +269,9 @@ class _CallPlan:
         self.undescribed = tuple({n for _, n in slots} - set(shapes))  # tensors that io_spec does not name
 
     def of(self, lowered) -> bool:
-        return (self.io_spec is lowered.io_spec and self.call_args is lowered.call_args
+        return (self.io_spec is lowered.io_spec
+                and ((self.fixed and self.call_args is lowered.call_args)
+                     or self.seen == tuple((kind, v) for kind, v in lowered.call_args))
                 and self.kernel_id == lowered.kernel_id and self.bindings is lowered.bindings
                 and self.bound == lowered.bindings and self.spec == lowered.io_spec["tensors"])
 

@@ -91,3 +91,18 @@ def test_an_argument_outside_the_io_spec_is_passed(calls):
                               call_args=(*k.call_args, ("tensor", "extra")))
     launch_lowered(lowered, b)
     assert calls[0][-2] == b["extra"].data_ptr()
+
+
+def test_call_args_changed_in_place_are_seen(calls):
+    k, b = _kernel(), _buffers()
+    for make in (list, lambda a: tuple(list(x) for x in a)):  # a list of pairs, a tuple of lists
+        lowered = SimpleNamespace(io_spec=k.io_spec, bindings=k.bindings, kernel_id=k.kernel_id,
+                                  call_args=make(k.call_args))
+        launch_lowered(lowered, b)
+        at = [i for i, (kind, _) in enumerate(lowered.call_args) if kind == "i64"][0]
+        if isinstance(lowered.call_args, list):
+            lowered.call_args[at] = ("i64", 3)
+        else:
+            lowered.call_args[at][1] = 3
+        launch_lowered(lowered, b)
+        assert calls[-2][at] == 5 and calls[-1][at] == 3
