@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import copy
 import ctypes
+import functools
 import threading
 from pathlib import Path
 from typing import Any, Dict, Iterable, Mapping, Optional, Sequence, Tuple
@@ -175,11 +176,16 @@ def _torch():
     return torch
 
 
-def torch_dtype(dtype: str):
+@functools.lru_cache(maxsize=None)
+def _torch_dtypes() -> Dict[str, Any]:
     import torch  # noqa: PLC0415
     return {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32, "f64": torch.float64,
             "i8": torch.int8, "i16": torch.int16, "u8": torch.uint8, "bool": torch.bool, "i1": torch.bool,
-            "i32": torch.int32, "i64": torch.int64}[dtype]
+            "i32": torch.int32, "i64": torch.int64}
+
+
+def torch_dtype(dtype: str):
+    return _torch_dtypes()[dtype]
 
 
 def to_device(arr: np.ndarray, dtype: str, device: str = "cuda"):
@@ -218,6 +224,15 @@ def tensor_shapes(io_spec: Mapping[str, Any], bindings: Mapping[str, Any]) -> Di
     return {n: tuple(resolve_dim(d, bindings) for d in spec["shape"]) for n, spec in io_spec["tensors"].items()}
 
 
+def _tensors_copy(tensors: Mapping[str, Any]) -> Any:
+    """io_spec["tensors"] as it is now, to compare with later: dtype and shape copied, dims that are
+    names or numbers as they are (a full deep copy is half of a plan's cost)."""
+    if type(tensors) is dict and all(type(s) is dict and all(type(d) in (str, int) for d in s["shape"])
+                                     for s in tensors.values()):
+        return {n: {**s, "shape": copy.copy(s["shape"])} for n, s in tensors.items()}
+    return copy.deepcopy(tensors)
+
+
 class _CallPlan:
     """What every launch of one lowered kernel shares, worked out once: the tensors' torch dtypes and
     bound shapes, the entry point, and the C arguments that are not pointers.  Nothing of a buffer is
@@ -229,11 +244,8 @@ class _CallPlan:
     def __init__(self, lowered) -> None:
         self.io_spec, self.bindings = lowered.io_spec, lowered.bindings
         self.bound = dict(lowered.bindings)
-        self.spec = copy.deepcopy(lowered.io_spec["tensors"])
+        self.spec = _tensors_copy(lowered.io_spec["tensors"])
         self.call_args, self.kernel_id = lowered.call_args, lowered.kernel_id
-        # pairs that cannot change under the plan are recognised by the tuple that holds them
-        self.fixed = type(self.call_args) is tuple and all(type(a) is tuple for a in self.call_args)
-        self.seen = tuple((kind, v) for kind, v in self.call_args)
         shapes = tensor_shapes(lowered.io_spec, lowered.bindings)
         self.tensors = tuple((n, spec["dtype"], torch_dtype(spec["dtype"]), shapes[n])
                              for n, spec in lowered.io_spec["tensors"].items())
@@ -241,7 +253,10 @@ class _CallPlan:
         args: list = []
         slots, workspaces = [], []
         self.program = None
-        for kind, v in lowered.call_args:
+        fixed = type(self.call_args) is tuple
+        for pair in self.call_args:
+            fixed = fixed and type(pair) is tuple
+            kind, v = pair
             if kind == "tensor":
                 slots.append((len(args), v))
                 args.append(None)
@@ -266,12 +281,14 @@ class _CallPlan:
                 raise HipRuntimeError(f"unknown call argument kind {kind}")
         args.append(None)  # the stream
         self.args, self.ptr_slots, self.workspaces = args, tuple(slots), tuple(workspaces)
-        self.undescribed = tuple({n for _, n in slots} - set(shapes))  # tensors that io_spec does not name
+        self.undescribed = tuple([n for _, n in slots if n not in shapes])  # tensors that io_spec does not name
+        # pairs that cannot change under the plan are recognised by the tuple that holds them
+        self.fixed, self.seen = fixed, None if fixed else tuple((kind, v) for kind, v in self.call_args)
 
     def of(self, lowered) -> bool:
         return (self.io_spec is lowered.io_spec
-                and ((self.fixed and self.call_args is lowered.call_args)
-                     or self.seen == tuple((kind, v) for kind, v in lowered.call_args))
+                and (self.call_args is lowered.call_args if self.fixed
+                     else self.seen == tuple((kind, v) for kind, v in lowered.call_args))
                 and self.kernel_id == lowered.kernel_id and self.bindings is lowered.bindings
                 and self.bound == lowered.bindings and self.spec == lowered.io_spec["tensors"])
 

@@ -106,3 +106,22 @@ def test_call_args_changed_in_place_are_seen(calls):
             lowered.call_args[at][1] = 3
         launch_lowered(lowered, b)
         assert calls[-2][at] == 5 and calls[-1][at] == 3
+
+
+@pytest.mark.parametrize("dim", ["N", {"kind": "const", "value": 96}])
+def test_io_spec_changed_in_place_is_seen(calls, dim):
+    """A dtype, a dim in a shape, or something inside a dim that is neither a name nor a number."""
+    plain = _kernel().io_spec["tensors"]["input_ptr"]
+    tensors = {"input_ptr": {"dtype": "f32", "shape": [5, 96]}, "output_ptr": dict(plain)}
+    spec = runtime._tensors_copy(tensors)
+    assert spec == tensors
+    tensors["input_ptr"]["shape"][1] = 97
+    assert spec != tensors
+    spec = runtime._tensors_copy(tensors)
+    tensors["output_ptr"]["dtype"] = "f16"
+    assert spec != tensors
+    tensors["output_ptr"]["shape"] = [dim]
+    spec = runtime._tensors_copy(tensors)
+    if isinstance(dim, dict):
+        dim["value"] = 7
+        assert spec != tensors
