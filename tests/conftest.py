@@ -15,6 +15,15 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a ROCm device and the built libintentir_hip.so")
 
 
+@pytest.hookimpl(tryfirst=True)  # before -m selects
+def pytest_collection_modifyitems(items):
+    """A test that uses the ``hip`` fixture is a GPU test, whether it says so or not: without the
+    marker neither ``-m gpu`` nor ``-m "not gpu"`` would run it."""
+    for item in items:
+        if "hip" in getattr(item, "fixturenames", ()):
+            item.add_marker(pytest.mark.gpu)
+
+
 def hip_ready() -> bool:
     """A ROCm device is visible (GPU tests fail loudly if the library is then missing)."""
     if os.environ.get("IHIP_FORCE_NO_GPU"):

@@ -90,6 +90,7 @@ def test_flat_form_equals_the_interpreter_kernel(hip, shape, types):
             assert torch.equal(got[EW_MODE_NATIVE][n], got[EW_MODE_INTERP][n]), f"{n} differs"
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dt,V", [("f32", 4), ("bf16", 8), ("i32", 4)])
 @pytest.mark.parametrize("total", [9, 64, 65, 67, 129, 257, 1025])  # in runs of V, and 1 or 3 elements more
 def test_flat_form_in_place(hip, dt, V, total):
