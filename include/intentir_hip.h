@@ -402,9 +402,10 @@ int ihip_elementwise_mode(int mode);
 /* Compile the native code of a program for the given operand types ahead of its first launch
  * (for example before capturing a graph).  Needs no device.  Checks the program like
  * ihip_elementwise_program; returns IHIP_OK, or an error whose message holds the compiler log.
- * The generated code fixes each operand's access form, so this prepares the form that dense
- * operands select: every input and output 16-byte aligned, read and written in full vectors
- * (inner size a multiple of 8 elements when all operands are 16-bit or narrower, else of 4).
+ * The generated code fixes each operand's access form, so this prepares the two forms that dense
+ * operands select (by row length): every input and output 16-byte aligned, read and written in
+ * full vectors (inner size a multiple of 8 elements when all operands are 16-bit or narrower, else
+ * of 4).
  * Other layouts (broadcast scalars and [M,1] columns, strided or unaligned operands, operands
  * read across their unit-stride axis such as a transpose) compile on their first launch, or
  * ahead of it through ihip_elementwise_prepare_operands. */

@@ -1173,8 +1173,9 @@ bool compile_checked(const JitForm& form, std::string* why) {
 }  // namespace
 
 // Compile (once) the native code of a validated program for the given operand types, in the
-// form that dense operands select (every input and output read and written in full-width
-// vectors); no device is needed.  Returns false with *why set when compilation fails.
+// forms that dense operands select (every input and output read and written in full-width
+// vectors): the row form, and the flat form that short rows take (plan_flat); no device is needed.
+// Returns false with *why set when compilation fails.
 bool prepare_elementwise_jit(const ihip_ew_instr* code, int n_code, int n_inputs, const int* in_dt, int n_outputs,
                              const int* out_dt, std::string* why) {
   const char w = ew_jit_width(n_inputs, in_dt, n_outputs, out_dt) == 8 ? '8' : '4';
@@ -1185,6 +1186,12 @@ bool prepare_elementwise_jit(const ihip_ew_instr* code, int n_code, int n_inputs
   f.n_outputs = n_outputs;
   for (int k = 0; k < n_inputs; ++k) f.in_dt[k] = in_dt[k], f.in_kind[k] = w;
   for (int k = 0; k < n_outputs; ++k) f.out_dt[k] = out_dt[k], f.out_kind[k] = w;
+  if (!compile_checked(f, why)) return false;
+  for (int pc = 0; pc < n_code; ++pc)
+    if (code[pc].op == IHIP_EW_IOTA) return true;
+  f.flat = true;
+  for (int k = 0; k < n_inputs; ++k) f.in_kind[k] = 'u';
+  for (int k = 0; k < n_outputs; ++k) f.out_kind[k] = 'u';
   return compile_checked(f, why);
 }
 

@@ -275,6 +275,39 @@ def test_native_code_compiles_for_launch_operands(name, ir, bindings, gen, misal
     assert st == 0, lib.ihip_last_error().decode()
 
 
+@pytest.mark.parametrize("dt,shapes", [("f32", [(1000, 64), (1000, 1024), (300, 1040), (257, 4)]),
+                                       ("bf16", [(1000, 200), (1000, 4096), (64, 8)])])
+def test_prepare_covers_dense_operands(dt, shapes):
+    """After ihip_elementwise_prepare, a launch on dense aligned operands whose inner size is a whole
+    number of vectors compiles nothing, in whichever form the length of its rows selects: what such
+    a launch runs is ready (prepare_operands returns in microseconds, a compile takes 0.1 s or more)."""
+    import random
+    import time
+
+    from intent_ir_amd.ewprogram import DTYPE_CODE, EwProgram
+    from intent_ir_amd.runtime import EwInstr, ew_program_args, load_library
+
+    lib = load_library()
+    scale = random.Random(time.time_ns()).uniform(1.0, 2.0)  # a program that no other test compiled
+    ops = ((OP["load"], 0, 0, 0, 0, 0.0), (OP["load"], 1, 1, 0, 0, 0.0), (OP["imm"], 2, 0, 0, 0, scale),
+           (OP["mul"], 3, 0, 2, 0, 0.0), (OP["add"], 3, 3, 1, 0, 0.0), (OP["store"], 0, 3, 0, 0, 0.0))
+    code = (EwInstr * len(ops))()
+    for i, (o, d, a, b, c, imm) in enumerate(ops):
+        code[i].op, code[i].dst, code[i].a, code[i].b, code[i].c, code[i].imm = o, d, a, b, c, imm
+    ind, outd = (ctypes.c_int32 * 2)(*[DTYPE_CODE[dt]] * 2), (ctypes.c_int32 * 1)(DTYPE_CODE[dt])
+    t0 = time.perf_counter()
+    assert lib.ihip_elementwise_prepare(code, len(ops), ind, 2, outd, 1) == 0, lib.ihip_last_error().decode()
+    compiled = time.perf_counter() - t0
+    for M, N in shapes:
+        st = (M * N, M * N, N, 1)
+        prog = EwProgram(ops, (("a", st), ("b", st)), ("y",), (M, N))
+        args = ew_program_args(prog, {"a": 0x100000, "b": 0x200000, "y": 0x300000}, dict.fromkeys("aby", dt))
+        t0 = time.perf_counter()
+        assert lib.ihip_elementwise_prepare_operands(*args[:8]) == 0, lib.ihip_last_error().decode()
+        took = time.perf_counter() - t0
+        assert took < compiled / 10, f"[{M}, {N}] compiled anew: {took:.3f} s"
+
+
 def test_prepare_rejects_bad_programs():
     from intent_ir_amd.runtime import EwInstr, load_library
 
