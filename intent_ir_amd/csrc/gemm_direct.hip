@@ -238,10 +238,12 @@ __global__ __launch_bounds__(64 * W) void gemm_bf16_direct(const uint16_t* __res
     load(slab, s0);
     for (int64_t i = s0; i < s1; ++i) {
       D::stage(slab, stage, lane);
+      __builtin_amdgcn_wave_barrier();  // rows staged by other lanes; a wave's LDS accesses stay in order
       if constexpr (kNT) {
         if (i + 1 < s1) load(slab, i + 1);
       }
       D::multiply(slab.b, stage, lane, acc);
+      __builtin_amdgcn_wave_barrier();  // before the next slab, or the sums, take their place
       if constexpr (!kNT) {
         if (i + 1 < s1) load(slab, i + 1);
       }
