@@ -150,6 +150,7 @@ __global__ __launch_bounds__(256) void pack_rows_kc(const uint16_t* __restrict__
 // Reads go along src rows, 16 bytes per lane at the row's own 2-byte boundary, writes along dst
 // rows in 16-byte stores, 8 lanes per 128-byte row piece.
 constexpr int kT = 64;
+typedef uint32_t u32_pair __attribute__((may_alias));  // two elements of the tile
 __global__ __launch_bounds__(256) void pack_rows_km(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                     int64_t R, int64_t K, int64_t K8) {
   __shared__ __attribute__((aligned(4))) uint16_t tile[kT][kT + 2];
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(256) void pack_rows_km(const uint16_t* __restrict__
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) *reinterpret_cast<uint32_t*>(&tile[32 * p + (threadIdx.x >> 3)][c + 2 * e]) = v[p][e];
+    for (int e = 0; e < 4; ++e) *reinterpret_cast<u32_pair*>(&tile[32 * p + (threadIdx.x >> 3)][c + 2 * e]) = v[p][e];
   __syncthreads();
   // write: dst row r0 + i gets k0 .. k0+63 (zeros past K; K8, a multiple of 8, may end inside
   // the tile), 8 columns per lane
