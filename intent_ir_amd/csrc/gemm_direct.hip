@@ -45,16 +45,13 @@ struct DirectPlan {
 namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef uint32_t u32_b2 __attribute__((aligned(2)));
 
 constexpr int kStep = 32;  // k per MFMA
 
-// 2 * NF bytes from any 2-byte boundary into NF / 2 dwords.
+// 2 * NF bytes (NF = 4 or 8) from any 2-byte boundary into NF / 2 dwords.
 template <int NF>
 __device__ __forceinline__ void load_cols(const uint16_t* p, uint32_t* d) {
-  if constexpr (NF == 2) {
-    d[0] = *reinterpret_cast<const u32_b2*>(p);
-  } else if constexpr (NF == 4) {
+  if constexpr (NF == 4) {
     const u32x2 v = *reinterpret_cast<const u32x2_b2*>(p);
     d[0] = v.x;
     d[1] = v.y;
@@ -312,14 +309,14 @@ hipError_t launch(const uint16_t* A, const uint16_t* B, const float* bias, uint1
 template <int MF, bool kNT>
 hipError_t launch_nf(const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, int64_t M, int64_t N,
                      int64_t K, int relu, const DirectPlan& p, float* P, int64_t ldp, hipStream_t s) {
-  if constexpr (!kNT && MF <= 2) {
+  if constexpr (kNT) {
+    if (p.nf == 2) return p.wk == 8 ? launch<MF, 2, kNT, 8>(A, B, bias, C, M, N, K, relu, p, P, ldp, s)
+                                    : launch<MF, 2, kNT, 4>(A, B, bias, C, M, N, K, relu, p, P, ldp, s);
+  } else if constexpr (MF <= 2) {
     if (p.nf == 8) return p.wk == 8 ? launch<MF, 8, kNT, 8>(A, B, bias, C, M, N, K, relu, p, P, ldp, s)
                                     : launch<MF, 8, kNT, 4>(A, B, bias, C, M, N, K, relu, p, P, ldp, s);
   }
-  if (p.wk == 8)
-    return p.nf == 2 ? launch<MF, 2, kNT, 8>(A, B, bias, C, M, N, K, relu, p, P, ldp, s)
-                     : launch<MF, 4, kNT, 8>(A, B, bias, C, M, N, K, relu, p, P, ldp, s);
-  return p.nf == 2 ? launch<MF, 2, kNT, 4>(A, B, bias, C, M, N, K, relu, p, P, ldp, s)
+  return p.wk == 8 ? launch<MF, 4, kNT, 8>(A, B, bias, C, M, N, K, relu, p, P, ldp, s)
                    : launch<MF, 4, kNT, 4>(A, B, bias, C, M, N, K, relu, p, P, ldp, s);
 }
 

@@ -316,9 +316,9 @@ static int64_t f32_tiles_ns(int64_t wgs, int64_t k) {
   return (wgs / 1024 * kF32NsPerK[4] + kF32NsPerK[(wgs % 1024 + 255) / 256]) * k;
 }
 
-static F32Split f32_split_plan(int64_t M, int64_t N, int64_t K, int tile) {
+static F32Split f32_split_plan(int64_t M, int64_t N, int64_t K) {
   F32Split best = {1, K};
-  if (M <= 0 || N <= 0 || (tile != 0 ? tile : gemm_f32_tile_extent(M, N)) != 64) return best;
+  if (M <= 0 || N <= 0 || gemm_f32_tile_extent(M, N) != 64) return best;
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64), ldp = (N + 3) / 4 * 4;
   int64_t best_ns = f32_tiles_ns(tiles, K);
   for (int64_t S = 2; S <= 32 && S * 128 <= K; ++S) {
@@ -331,7 +331,7 @@ static F32Split f32_split_plan(int64_t M, int64_t N, int64_t K, int tile) {
 
 // Workspace bytes of ihip_gemm_f32_bias_relu_ws: the planes of partial sums, 0 where K is not split.
 int64_t gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-  const F32Split sp = f32_split_plan(M, N, K, 0);
+  const F32Split sp = f32_split_plan(M, N, K);
   return sp.S > 1 ? sp.S * M * ((N + 3) / 4 * 4) * 4 : 0;
 }
 
@@ -349,7 +349,7 @@ hipError_t launch_gemm_f32_bias_relu(const float* A, const float* B, const float
   const int tb_ext = tile != 0 ? tile : gemm_f32_tile_extent(M, N);
   F32Split sp = {1, K};
   if (tile == 0 && ws != nullptr && al16(ws)) {
-    sp = f32_split_plan(M, N, K, 0);
+    sp = f32_split_plan(M, N, K);
     if (sp.S * M * ((N + 3) / 4 * 4) * 4 > ws_bytes) sp = {1, K};
   }
   float* P = static_cast<float*>(ws);

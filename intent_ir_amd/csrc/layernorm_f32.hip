@@ -301,8 +301,13 @@ static void launch_ln32_held(const float* x, const float* w, const float* b, flo
     else launch_ln32_grouped<64>(x, w, b, y, mean, rstd, M, N, eps, s);
     return;
   }
-  if (n4 <= 64) launch_ln32_wave<1, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);  // N < 4, or 257-259
-  else if (n4 <= 128) launch_ln32_wave<2, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+  if constexpr (kU) {
+    if (n4 <= 64) {  // N < 4, or 257-259
+      launch_ln32_wave<1, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
+      return;
+    }
+  }
+  if (n4 <= 128) launch_ln32_wave<2, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
   else if (n4 <= 256) launch_ln32_wave<4, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
   else if (n4 <= 512) launch_ln32_wave<8, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
   else if (n4 <= 1024) launch_ln32_wave<16, kU>(x, w, b, y, mean, rstd, M, n4, N, eps, s);
