@@ -1,6 +1,5 @@
-// C = act(A @ op(B) + bias) in bf16 for products with one small side (a few rows or a few columns:
-// the step of a decode, a narrow head) and for small products: A [M, K], B [K, N] or [N, K], any
-// alignment, f32 accumulation on v_mfma_f32_16x16x32_bf16, C bf16 (RNE).
+// C = act(A @ op(B) + bias) in bf16 for products of few rows (the step of a decode): A [M, K], M up to
+// 128, B [K, N] or [N, K], any alignment, f32 accumulation on v_mfma_f32_16x16x32_bf16, C bf16 (RNE).
 //
 // Such a product is bound by reading its long operand once (32 x 32000 x 4096: 262 MB of B for 8
 // GFLOP), and the tiled kernels spend it on rows they do not store, on a copy of ragged operands
@@ -19,14 +18,15 @@
 //  * the waves of a workgroup that share a block take consecutive ranges of K, add their sums in
 //    LDS in order, and each thread rounds and stores 4 consecutive columns.  (Taking the slabs in
 //    turn instead ran 32 x 32000 x 4096 10% slower: every wave then walks the same few channels.)
-//    Where the blocks leave CUs without a workgroup, segments of K go to workgroups of their own
-//    and their f32 sums, through a workspace, to the split-K reduction: one CU takes in 16-30 GB/s
-//    whatever its waves, so a product needs all of them.
-// Measured in us, tiled (packed, split) kernels -> this one: B as [N, K] 32 x 32000 x 4096 62.5 -> 51.9
-// (5.1 TB/s), 64 x 32000 x 4096 64.3 -> 60.1, 16 x 4096 x 4096 16.8 -> 12.8, 16 x 1024 x 8192 14.8 ->
-// 10.9, 1 x 8192 x 8192 41.1 -> 26.5; B as [K, N] 16 x 32000 x 4096 57.7 -> 48.9, 16 x 16384 x 2048 25.4
-// -> 18.7, 16 x 1024 x 8192 15.0 -> 11.4; ragged: 1 x 40274 x 4311 364 -> 76, 2 x 24482 x 4991 ([N, K])
-// 214 -> 68, 16 x 4097 x 4095 49.5 -> 21.2, 64 x 32001 x 1001 67.6 -> 34.0, 2 x 117 x 1209 19.0 -> 7.
+//    Where the blocks are at most half the CUs, segments of K go to workgroups of their own, as many
+//    as keep them all in one round of 256, and their f32 sums, through a workspace, to the split-K
+//    reduction: one CU takes in 16-30 GB/s whatever its waves, so a product needs all of them.
+// Kernel times in us (graph replays), tiled (packed, split) kernels -> this one: B as [N, K]
+// 32 x 32000 x 4096 63.2 -> 51.8 (5.1 TB/s), 16 x 4096 x 4096 13.4 -> 10.8, 16 x 1024 x 8192 13.0 ->
+// 9.9, 1 x 8192 x 8192 38.0 -> 24.8; B as [K, N] 16 x 32000 x 4096 53.1 -> 49.0, 16 x 16384 x 2048 16.9
+// -> 14.2, 16 x 1024 x 8192 13.2 -> 10.5; ragged: 1 x 40274 x 4311 362.5 -> 82.4, 2 x 24482 x 4991
+// ([N, K]) 212.9 -> 66.2, 16 x 4097 x 4095 38.2 -> 12.6, 64 x 32001 x 1001 66.8 -> 27.4, 2 x 117 x
+// 1209 16.2 -> 7.8.
 // Every C element sums its k in ascending slabs of 32 as the tiled kernels do: with one wave along
 // K the bits are theirs, with more the result differs by the f32 summation order only.  The split
 // depends on M, N, K and B's layout, so alignment does not change a bit.
@@ -334,10 +334,11 @@ hipError_t launch_mf(const uint16_t* A, const uint16_t* B, const float* bias, ui
 
 // Waves along K and segments of a product whose blocks are 64 columns wide: waves until 2048 run
 // (8 per CU) or each has two slabs; then, where the launch and the round trip of a reduction (3-4
-// us) are less than what idle CUs cost, segments until every CU has a workgroup.  B as [N, K] with
-// more than 64 blocks runs 32-column blocks on every CU instead (1 x 8192 x 8192: 26.5 us, in two
-// segments 30.0); columns of B as [K, N] that narrow would be read half a line at a time (40.3
-// against 32.7).
+// us) are less than what idle CUs cost, as many segments as 256 workgroups allow.  (Rounded up they
+// made 257 to 300, a second round for a few: 3 x 3200 x 12736 23.9 us, now 17.9; 16 x 1856 x 14024
+// ([N, K]) 25.7, now 16.5.)  B as [N, K] with more than 64 blocks runs 32-column blocks on every CU
+// instead (1 x 8192 x 8192: 26.5 us, in two segments 30.0); columns of B as [K, N] that narrow would
+// be read half a line at a time (40.3 against 32.7).
 DirectPlan gemm_direct_plan(int64_t M, int64_t N, int64_t K, bool transpose_b) {
   DirectPlan p;
   p.mf = M <= 16 ? 1 : M <= 32 ? 2 : 4;
@@ -346,27 +347,68 @@ DirectPlan gemm_direct_plan(int64_t M, int64_t N, int64_t K, bool transpose_b) {
   while (p.wk < 8 && blocks * p.wk < 2048 && K >= 256 * p.wk) p.wk *= 2;
   p.S = 1;
   if (blocks <= (transpose_b ? 64 : 128) && K >= 2048) {
-    const int64_t fill = (256 + blocks - 1) / blocks, most = K / 512;
+    const int64_t fill = 256 / blocks, most = K / 512;
     p.S = static_cast<int>(fill < most ? (fill < 16 ? fill : 16) : (most < 16 ? most : 16));
   }
   p.nf = 4;
   return p;
 }
 
-// Where this kernel is taken: K above two slabs, 16 to 65536 columns (wider products fill the
-// tiled kernels: 5.1 TB/s at 32 x 128256 x 4096), A and B below 2^31 elements (offsets are 32 bits).
-// Operands that the tiled kernels would have to copy first (rows off 16-byte alignment by their
-// length): up to 128 rows (beyond, the copy is repaid: 256 x 4097 x 4095 69 us here).  Operands they
-// read in place, up to 49152 columns: up to 64 rows of B as [N, K] (96 x 32000 x 4096: 80.6 against
-// 67.7); of B as [K, N], whose columns cost more loads, up to 16, and up to 32 where the blocks are
-// 128 columns wide or K is short (32 x 8192 x 8192 35.7 against 34.1, 64 x 32000 x 4096 77 against 54).
+// Where this kernel is taken: K above two slabs, 16 to 65536 columns, A and B below 2^31 elements
+// (offsets are 32 bits), and the side of the lines below on which it was the faster one.  The lines
+// come from 5900 shapes drawn over M <= 128, N <= 65536, K <= 20000 in both layouts and 700 of round
+// sizes, each timed here and on the kernels that run otherwise (tiled, packed or split) by graph
+// replays of both on the same buffers.  The 4500 drawn ones that are taken ran 1.69x faster (geometric
+// mean), nine of them slower by more than 3% (aligned ones by at most 8%); the others would have run
+// 1.15x slower here.  What the lines follow:
+//  * blocks of 64 columns (with the rows' blocks) against the 256 CUs: up to 256 run in one round (of
+//    half as wide ones, two); the second round of 257 to 512 is partly empty and pays for few rows or
+//    long K only;
+//  * K: a wave needs some slabs to hide its latency, the more the more rows it multiplies (B as [K, N],
+//    17 x 13888 x 136 9.0 against 5.3 us, 28 x 912 x 176 9.4 against 5.5);
+//  * operands off 16-byte alignment by their length, which the other kernels copy first: up to 128 rows.
 bool gemm_direct_takes(int64_t M, int64_t N, int64_t K, bool transpose_a, bool transpose_b) {
   if (transpose_a || M < 1 || N < 16 || N > 65536 || K <= 128) return false;
   if (N * K >= (int64_t(1) << 31) || M * K >= (int64_t(1) << 31)) return false;
-  if (K % 8 != 0 || (!transpose_b && N % 8 != 0)) return M <= 128;
-  if (N > 49152) return false;
-  if (transpose_b) return M <= 64;
-  return M <= 16 || (M <= 32 && (N >= 16384 || K <= 4096));
+  const bool ragged = K % 8 != 0 || (!transpose_b && N % 8 != 0);
+  if (M > (ragged ? 128 : transpose_b ? 64 : 32) || (!ragged && N > 49152)) return false;
+  const DirectPlan p = gemm_direct_plan(M, N, K, transpose_b);
+  const int64_t b = (M + 16 * p.mf - 1) / (16 * p.mf) * ((N + 63) / 64), w = b * p.S;
+  if (ragged && transpose_b) {
+    if (M <= 32) return true;
+    if (M <= 64) return K < 4096 || b <= 128 || b > 192;
+    if (K < 256) return b <= 256;
+    return K < 4096 || b <= 64 || b > 256 || (K < 8192 && (b <= 128 || b > 192));
+  }
+  if (ragged) {
+    if (M <= 16) return true;
+    if (M <= 32) return K >= 256 || b > 192;
+    if (M <= 64) return K >= 384 || b > 512 || (K >= 256 && b > 64);
+    return K >= 768 || (K >= 512 && b <= 256);
+  }
+  if (b > 512) return transpose_b ? M <= 32 || K >= 768 : M <= 16 || K < 2048;
+  // rows of B as [N, K] a multiple of 1 KiB apart, which the tiled kernels read more slowly
+  const bool pitch = transpose_b && K % 512 == 0;
+  if (b > 256) {
+    if (pitch && K >= 3072) return M <= 32 || (K >= 4096 && b > 352);
+    if (M > 32) return false;
+    if (M > 16) return K >= 4096 && b > (transpose_b ? 320 : 448);
+    if (K < (transpose_b ? 256 : 512) || (K >= 1024 && K < 2048)) return false;
+    return K < 1024 || (b > 320 && (K >= 4096 || !transpose_b));
+  }
+  if (pitch && M > 32) return K >= 512 && K <= 4096 && (b <= 128 || b > 192);
+  if (pitch && M > 16) return K >= 512 && (K < 8192 || b <= 128 || b > 170);
+  if (M <= 16) {
+    if (!transpose_b && (K < 256 || (K >= 4096 && b > 64 && b <= 85))) return false;
+    // workgroups launched, in rounds of 256: long K asks for rounds at least 5/8 full
+    const int64_t u = transpose_b && w < 256 ? 2 * w : w, rounds = (u + 255) / 256;
+    return K < 8192 || b <= 64 || u * 8 >= rounds * 256 * 5;
+  }
+  if (M <= 32) {
+    if (!transpose_b) return K >= 512 && K <= 4096;
+    return K >= 256 && (K < 2048 || b <= 64 || (b <= 128 && K < 8192) || (b > 192 && K < 4096));
+  }
+  return K >= 384 && (w < 64 || b <= 8 || (w <= 128 && K < 2560) || K < 1024);
 }
 
 int gemm_direct_segments(int64_t M, int64_t N, int64_t K, bool transpose_b) {

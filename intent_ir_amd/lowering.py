@@ -358,13 +358,55 @@ def gemm_direct_takes(M: int, N: int, K: int, ta: bool, tb: bool) -> bool:
     """gemm_direct.hip gemm_direct_takes."""
     if ta or M < 1 or not 16 <= N <= 65536 or K <= 128 or max(M, N) * K >= (1 << 31):
         return False
-    if K % 8 != 0 or (not tb and N % 8 != 0):
-        return M <= 128
-    if N > 49152:
+    ragged = K % 8 != 0 or (not tb and N % 8 != 0)
+    if M > (128 if ragged else 64 if tb else 32) or (not ragged and N > 49152):
         return False
-    if tb:
-        return M <= 64
-    return M <= 16 or (M <= 32 and (N >= 16384 or K <= 4096))
+    mf, _, S = gemm_direct_plan(M, N, K, tb)
+    b = _cdiv(M, 16 * mf) * _cdiv(N, 64)
+    w = b * S
+    if ragged and tb:
+        if M <= 32:
+            return True
+        if M <= 64:
+            return K < 4096 or b <= 128 or b > 192
+        if K < 256:
+            return b <= 256
+        return K < 4096 or b <= 64 or b > 256 or (K < 8192 and (b <= 128 or b > 192))
+    if ragged:
+        if M <= 16:
+            return True
+        if M <= 32:
+            return K >= 256 or b > 192
+        if M <= 64:
+            return K >= 384 or b > 512 or (K >= 256 and b > 64)
+        return K >= 768 or (K >= 512 and b <= 256)
+    if b > 512:
+        return (M <= 32 or K >= 768) if tb else (M <= 16 or K < 2048)
+    pitch = tb and K % 512 == 0
+    if b > 256:
+        if pitch and K >= 3072:
+            return M <= 32 or (K >= 4096 and b > 352)
+        if M > 32:
+            return False
+        if M > 16:
+            return K >= 4096 and b > (320 if tb else 448)
+        if K < (256 if tb else 512) or 1024 <= K < 2048:
+            return False
+        return K < 1024 or (b > 320 and (K >= 4096 or not tb))
+    if pitch and M > 32:
+        return 512 <= K <= 4096 and (b <= 128 or b > 192)
+    if pitch and M > 16:
+        return K >= 512 and (K < 8192 or b <= 128 or b > 170)
+    if M <= 16:
+        if not tb and (K < 256 or (K >= 4096 and 64 < b <= 85)):
+            return False
+        u = 2 * w if tb and w < 256 else w
+        return K < 8192 or b <= 64 or u * 8 >= _cdiv(u, 256) * 256 * 5
+    if M <= 32:
+        if not tb:
+            return 512 <= K <= 4096
+        return K >= 256 and (K < 2048 or b <= 64 or (b <= 128 and K < 8192) or (b > 192 and K < 4096))
+    return K >= 384 and (w < 64 or b <= 8 or (w <= 128 and K < 2560) or K < 1024)
 
 
 def gemm_direct_plan(M: int, N: int, K: int, tb: bool) -> Tuple[int, int, int]:
@@ -374,7 +416,7 @@ def gemm_direct_plan(M: int, N: int, K: int, tb: bool) -> Tuple[int, int, int]:
     wk = 1
     while wk < 8 and blocks * wk < 2048 and K >= 256 * wk:
         wk *= 2
-    S = min(_cdiv(256, blocks), K // 512, 16) if blocks <= (64 if tb else 128) and K >= 2048 else 1
+    S = min(256 // blocks, K // 512, 16) if blocks <= (64 if tb else 128) and K >= 2048 else 1
     return mf, wk, S
 
 

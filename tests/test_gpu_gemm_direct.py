@@ -21,7 +21,7 @@ GUARD = 64
 SHAPES = [(1, 16, 129), (15, 17, 191), (16, 63, 136), (17, 65, 193), (31, 64, 192), (32, 130, 200), (33, 66, 520),
           (64, 127, 1000), (65, 129, 327), (127, 71, 511), (128, 515, 263), (1, 1001, 2049), (7, 4097, 2056),
           (16, 1024, 8192), (48, 1000, 4104), (64, 300, 8191), (3, 16384, 136), (5, 28672, 2048), (20, 25601, 2100),
-          (2, 8200, 2304), (32, 33000, 160)]
+          (2, 8200, 2304), (32, 33000, 160), (17, 64, 512), (64, 512, 384), (65, 129, 771), (127, 71, 1023), (48, 392, 520)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES + [(64, 49152, 4096), (128, 65536, 999), (128, 263, 128), (16, 50256, 4096)])
