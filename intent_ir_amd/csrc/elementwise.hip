@@ -123,6 +123,10 @@ __global__ __launch_bounds__(256) void bias_gelu_axpy_bf16_vec(const u32x4* __re
 // shifted against each other.  Against an element per thread, us: [32768, 4099] 229.2 -> 88.8 (6.05
 // TB/s), [7744, 2397] 42.5 -> 14.7, [1000000, 23] 49.5 -> 19.0.  8 <= N, total < 2^31 - 2^13; magic, shift: floor(e / N) as
 // (e * magic) >> shift.
+// From kFlatMin elements on: of fewer its runs leave most CUs idle, and an element per thread is the
+// faster form (kernel times, one element -> runs: [1173, 82] 2.14 -> 3.14, [3328, 175] 2.53 -> 3.23;
+// over 2^20 to 2^21 elements 0.94 to 1.29x, over 2^21 to 2^22 1.05 to 1.59x faster).
+constexpr int64_t kFlatMin = int64_t(1) << 21;
 template <bool kFolded>
 __global__ __launch_bounds__(256) void bias_gelu_axpy_bf16_flat(const uint16_t* __restrict__ x,
                                                                 const uint16_t* __restrict__ bias,
@@ -216,7 +220,8 @@ hipError_t launch_bias_gelu_axpy_bf16(const uint16_t* x, const uint16_t* bias, u
       else
         bias_gelu_axpy_bf16_vec<kRows, false, false><<<grid, dim3(256), 0, s>>>(x8, b8, y8, M, n8, alpha, lanes);
     }
-  } else if (const int64_t total = M * N; N >= 8 && total < (int64_t(1) << 31) - (1 << 13)) {
+  } else if (const int64_t total = M * N;
+             N >= 8 && total >= kFlatMin && total < (int64_t(1) << 31) - (1 << 13)) {
     const int64_t wgs = (total + 8191) / 8192;
     int l = 0;  // ceil(log2 N): magic / 2^(31 + l) exceeds 1 / N by less than 2^-31 / N
     while ((int64_t(1) << l) < N) ++l;

@@ -965,7 +965,8 @@ def _match_gelu_axpy(c: _Ctx) -> Optional[HipLoweredKernel]:
         launch = HipLaunch((max(1, _cdiv(N // 8, lanes)), max(1, min(65535, _cdiv(M, 8 * (256 // lanes)))), 1),
                            (256, 1, 1), 0)
     else:
-        per = 8192 if N >= 8 and M * N < (1 << 31) - (1 << 13) else 256  # runs of 8 elements, or one a thread
+        # runs of 8 elements, or one a thread
+        per = 8192 if N >= 8 and (1 << 21) <= M * N < (1 << 31) - (1 << 13) else 256
         launch = HipLaunch((max(1, min(65536, _cdiv(M * N, per))), 1, 1), (256, 1, 1), 0)
     return HipLoweredKernel(c.fn.name, "ihip_bias_gelu_tanh_axpy_bf16", c.io([x, bias, oname]), launch, [oname],
                             dict(c.b), (("tensor", x), ("tensor", bias), ("tensor", oname), ("i64", M), ("i64", N),

@@ -70,7 +70,7 @@ def test_any_split_over_bytes(hip, M, N, off):
 
 
 @pytest.mark.parametrize("M,N", [(1, 8), (1, 9), (3, 9), (5, 15), (700, 8), (301, 17), (40, 257), (9, 1603), (3, 4099),
-                                 (2000, 23)])
+                                 (2000, 23), (233017, 9), (123362, 17), (1309, 1603), (1, 2097167)])
 @pytest.mark.parametrize("ox,ob,oy", [(0, 0, 0), (1, 0, 0), (3, 5, 7), (0, 1, 4)])
 @pytest.mark.parametrize("alpha", [0.5, 0.0])
 def test_gelu_rows_at_any_2_byte_boundary(hip, M, N, ox, ob, oy, alpha):
@@ -102,7 +102,8 @@ def test_gelu_rows_at_any_2_byte_boundary(hip, M, N, ox, ob, oy, alpha):
     assert (h[:oy] == 0x1234).all() and (h[oy + M * N:] == 0x1234).all(), "written outside y"
 
 
-@pytest.mark.parametrize("M,N", [(1, 9), (1, 513), (3, 171), (1, 2049), (1, 8193), (7, 1171), (5, 1639), (683, 771)])
+@pytest.mark.parametrize("M,N", [(1, 9), (1, 513), (3, 171), (1, 2049), (1, 8193), (7, 1171), (5, 1639), (683, 771),
+                                 (1, 2097161), (233019, 9), (1031, 2049), (2049, 1025)])
 def test_gelu_in_place(hip, M, N):
     """y may be x: the runs at the end, which share elements across waves and workgroups, included."""
     import torch
