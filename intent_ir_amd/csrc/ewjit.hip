@@ -986,22 +986,24 @@ struct JitPlan {
 // every output and input is one value per element of the iteration space in memory order, per
 // column, per row or one for all (no iota: a run has no single row), and the space has at least
 // one run and less than 2^31 elements.  It is taken when the row form would leave an operand
-// without full vectors (D3 % V != 0, or a base off its vector's alignment: `vectors` false), 30%
-// of the lanes of the waves that a row occupies idle, or, for rows of several workgroups, a quarter
-// of their lanes.  Measured in us, row form -> flat form: without vectors, bf16 sigmoid [4096, 12289]
-// 126.6 -> 38.0 (5.3 TB/s), [1000000, 23] 627.8 -> 19.9, f32 bias + ReLU [8192, 4099] 83.4 -> 52.0,
-// [65536, 257] 49.2 -> 27.5, [262144, 24] 37.9 -> 11.2; idle lanes, f32 [400000, 64] 59.6 -> 35.2,
-// [150000, 168] (66% of a wave) 37.1 -> 36.3, [60000, 1040] (51% of two workgroups) 108.3 -> 84.3,
-// bf16 [100000, 200] 28.2 -> 18.0, [40000, 1040] 37.2 -> 33.0, [8192, 2600] 22.3 -> 19.2; on the
-// other side f32 [100000, 200] (78%) 29.7 -> 30.2, [60000, 512] 41.4 -> 43.5, [8192, 8192] 85.2 -> 89.0,
-// bf16 [20000, 4096] 58.6 -> 60.2.
+// without full vectors (D3 % V != 0, or a base off its vector's alignment: `vectors` false), or lanes
+// idle: 30% of those of the waves that a row occupies, or, for rows of several workgroups, a quarter
+// of theirs.  4-byte operands that move 16 MB or more are bound by memory sooner, and the lines lie
+// lower: rows of one wave 45% (16-80 MB; 30% above), of up to four 100% and 45%, workgroups 3/8 and a
+// quarter.  A space of one row is left to the row form where that moves 4 elements at a time (`quads`):
+// there is no second row for the idle lanes to take.  Measured in us, row form -> flat form: without
+// vectors, bf16 sigmoid [4096, 12289] 126.6 -> 38.0 (5.3 TB/s), [1000000, 23] 627.8 -> 19.9, f32 bias +
+// ReLU [8192, 4099] 83.4 -> 52.0, [65536, 257] 49.2 -> 27.5, [262144, 24] 37.9 -> 11.2; idle lanes, f32
+// [400000, 64] 59.6 -> 35.2, [60000, 1040] (51% of two workgroups) 108.3 -> 84.3, bf16 [100000, 200]
+// 28.2 -> 18.0, [40000, 1040] 37.2 -> 33.0, [8192, 2600] 22.3 -> 19.2; on the other side f32 [34161, 168]
+// (66% of a wave, 46 MB) 10.2 -> 10.8, [28208, 280] (55% of two, 63 MB) 13.2 -> 14.2, [2017, 2280] (74%
+// of three workgroups, 37 MB) 8.8 -> 9.7, [60000, 512] 41.4 -> 43.5, [8192, 8192] 85.2 -> 89.0, bf16
+// [20000, 4096] 58.6 -> 60.2, [1, 4544] 2.4 -> 2.7.
 bool plan_flat(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inputs, int n_inputs,
-               const int64_t (&shape)[4], bool vectors, int V, JitPlan& pl) {
+               const int64_t (&shape)[4], bool vectors, bool quads, int V, JitPlan& pl) {
   EwJitArgs& a = pl.a;
   const int64_t D3 = shape[3], total = a.rows * D3;
-  const int64_t wave_lanes = (a.nvec + 63) / 64 * 64, wg_lanes = (a.nvec + 255) / 256 * 256;
-  const bool idle = a.nvec * 10 < wave_lanes * 7 || (a.nvec > 256 && a.nvec * 4 < wg_lanes * 3);
-  if (total < V || total >= (int64_t(1) << 31) - 256 * 4 * 8 || (vectors && !idle)) return false;
+  if (total < V || total >= (int64_t(1) << 31) - 256 * 4 * 8 || (a.rows == 1 && quads)) return false;
   for (int pc = 0; pc < n_code; ++pc)
     if (code[pc].op == IHIP_EW_IOTA) return false;
   char kind[IHIP_EW_NATIVE_MAX_INPUTS + 1] = {};
@@ -1017,6 +1019,15 @@ bool plan_flat(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inp
     else if (is(3, 0) && is(2, 1) && is(1, r2) && is(0, r1)) kind[k] = per_row;
     else return false;
   }
+  const auto esize = [](int dt) -> int64_t { return dt == IHIP_DT_F32 || dt == IHIP_DT_I32 ? 4 : dt == IHIP_DT_BOOL ? 1 : 2; };
+  int64_t bytes = 0;  // of the operands that are one value per element
+  for (int k = 0; k < n_inputs; ++k) bytes += kind[k] == 'u' ? esize(pl.form.in_dt[k]) * total : 0;
+  for (int k = 0; k < pl.form.n_outputs; ++k) bytes += esize(pl.form.out_dt[k]) * total;
+  const bool big = V == 4 && bytes >= 16000000, mid = big && bytes < 80000000;
+  const int64_t wave_lanes = (a.nvec + 63) / 64 * 64, wg_lanes = (a.nvec + 255) / 256 * 256;
+  const int64_t twentieths = a.nvec <= 64 ? (mid ? 11 : 14) : mid ? 0 : big ? 11 : 14;
+  const bool idle = a.nvec * 20 < wave_lanes * twentieths || (a.nvec > 256 && a.nvec * 8 < wg_lanes * (mid ? 5 : 6));
+  if (vectors && !idle) return false;
   a.total = static_cast<uint32_t>(total);
   // floor(e / D3) for e < 2^31: with l = ceil(log2 D3), magic = floor(2^(31+l) / D3) + 1 exceeds
   // 2^(31+l) / D3 by at most 1, so (e * magic) / 2^(31+l) exceeds e / D3 by at most e / 2^(31+l) <
@@ -1136,10 +1147,16 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
   }
   if (tile_mask == 0) {
     const char full = V == 8 ? '8' : '4';
-    bool vectors = true;
-    for (int k = 0; k < n_inputs; ++k) vectors &= in_kind[k] == full || in_kind[k] == 'b';
-    for (int k = 0; k < n_outputs; ++k) vectors &= out_kind[k] == full;
-    if (plan_flat(code, n_code, inputs, n_inputs, shape, vectors, V, pl)) return true;
+    bool vectors = true, quads = true;
+    for (int k = 0; k < n_inputs; ++k) {
+      vectors &= in_kind[k] == full || in_kind[k] == 'b';
+      quads &= in_kind[k] != 's';
+    }
+    for (int k = 0; k < n_outputs; ++k) {
+      vectors &= out_kind[k] == full;
+      quads &= out_kind[k] != 's';
+    }
+    if (plan_flat(code, n_code, inputs, n_inputs, shape, vectors, quads, V, pl)) return true;
   }
   f.rowinv = rowinv;
   if (tile_mask != 0) {  // one workgroup per 64 x 64 tile, at most one per 128 x 32 (linear id; grid-strided

@@ -1113,7 +1113,7 @@ def _ew_launch(prog, dtype_of) -> HipLaunch:
         tx, ty = _cdiv(sh[3], 64), sh[0] * sh[1] * _cdiv(sh[2], 64)
         return HipLaunch((max(1, min(tx, 65535)), max(1, min(ty, 65535)), 1), (256, 1, 1), tiled * 64 * 65 * 4)
     rows = sh[0] * sh[1] * sh[2]
-    flat = _ew_flat_workgroups(prog, sh, v)
+    flat = _ew_flat_workgroups(prog, sh, v, dtype_of)
     if flat:
         return HipLaunch((flat, 1, 1), (256, 1, 1), 0)
     gx = max(1, min(1024, _cdiv(_cdiv(sh[3], v), 256)))
@@ -1125,11 +1125,10 @@ def _ew_launch(prog, dtype_of) -> HipLaunch:
     return HipLaunch((gx, max(1, min(_cdiv(rows, U), 65535, _cdiv(16384, gx))), 1), (256, 1, 1), 0)
 
 
-def _ew_flat_workgroups(prog, sh, v: int) -> int:
+def _ew_flat_workgroups(prog, sh, v: int, dtype_of) -> int:
     """Workgroups of the flat form (ewjit.hip plan_flat), 0 where it is not taken: operands that are
     one value per element in memory order, per column, per row or one for all, no iota, and rows that
-    would leave an operand without full vectors, 30% of the lanes of its waves idle, or a quarter of
-    the lanes of several workgroups."""
+    would leave an operand without full vectors or too many lanes of its waves or workgroups idle."""
     d0, d1, d2, d3 = sh
     rows = d0 * d1 * d2
     total, nvec = rows * d3, _cdiv(d3, v)
@@ -1137,20 +1136,28 @@ def _ew_flat_workgroups(prog, sh, v: int) -> int:
     if iota or not v <= total < (1 << 31) - 8192:
         return 0
 
-    def full(st):  # whole V-element vectors in the row form, or one value along the row
-        return st[3] == 0 or (d3 % v == 0 and st[3] == 1 and all(st[d] % v == 0 or sh[d] == 1 for d in range(3)))
+    def vec(st, w):  # whole w-element vectors in the row form, or one value along the row
+        return st[3] == 0 or (d3 % w == 0 and st[3] == 1 and all(st[d] % w == 0 or sh[d] == 1 for d in range(3)))
 
-    vectors = d3 % v == 0 and all(full(st) for _, st in prog.inputs)
-    idle = nvec * 10 < _cdiv(nvec, 64) * 64 * 7 or (nvec > 256 and nvec * 4 < _cdiv(nvec, 256) * 256 * 3)
-    if vectors and not idle:
+    if rows == 1 and d3 % 4 == 0 and all(vec(st, 4) for _, st in prog.inputs):
         return 0
     forms = ((d1 * d2 * d3, d2 * d3, d3, 1), (0, 0, 0, 0), (0, 0, 0, 1), (d1 * d2, d2, 1, 0))
-    one = []  # inputs that are one value for all: not loaded per run
-    for _, st in prog.inputs:
+    one, moved = [], [n for n in prog.outputs]  # inputs that are one value for all: not loaded per run
+    for n, st in prog.inputs:
         f = next((i for i, want in enumerate(forms) if all(sh[d] == 1 or st[d] == want[d] for d in range(4))), None)
         if f is None:
             return 0
         one.append(f == 1)
+        if f == 0:
+            moved.append(n)
+    nbytes = total * sum({"f32": 4, "i32": 4, "bool": 1, "i1": 1, "u8": 1}.get(dtype_of(n), 2) for n in moved)
+    big = v == 4 and nbytes >= 16000000
+    mid = big and nbytes < 80000000
+    share = (11 if mid else 14) if nvec <= 64 else 0 if mid else 11 if big else 14
+    idle = (nvec * 20 < _cdiv(nvec, 64) * 64 * share
+            or (nvec > 256 and nvec * 8 < _cdiv(nvec, 256) * 256 * (5 if mid else 6)))
+    if d3 % v == 0 and all(vec(st, v) for _, st in prog.inputs) and not idle:
+        return 0
     loads = sum(1 for ins in prog.code if ins[0] == 1 and not one[ins[2]])
     u = 4 if loads == 0 else max(1, min(4, 64 // (loads * v)))
     return min(65536, _cdiv(total, 256 * v * u))

@@ -19,7 +19,8 @@ CODE = ((OP["load"], 0, 0, 0, 0, 0.0), (OP["load"], 1, 1, 0, 0, 0.0), (OP["load"
 # says whether dense operands at aligned bases take the flat form (f32: 4 elements a run)
 SHAPES = [((1,), False), ((3,), False), ((5,), True), ((4099,), True), ((7, 1), True), ((1000, 3), True), ((33, 4), True),
           ((257, 7), True), ((300, 8), True), ((129, 24), True), ((77, 257), True), ((5, 1021), True), ((9, 1024), False),
-          ((64, 1000), False), ((3, 4, 65), True), ((2, 3, 5, 17), True), ((2, 1, 3, 1030), True)]
+          ((64, 1000), False), ((3, 4, 65), True), ((2, 3, 5, 17), True), ((2, 1, 3, 1030), True), ((96,), False), ((1, 2280), False),
+          ((2000, 280), True)]
 KINDS = ("dense", "column", "row", "scalar")
 
 
@@ -44,6 +45,17 @@ def test_flat_form_is_taken_for_short_and_ragged_rows(shape, flat):
     if len(shape) == 4:
         src = elementwise_source(_program(shape, ("dense", "outer", "dense"))[0], ptrs, types)
         assert "ldf<0, 'u'>(a.in" not in src
+
+
+@pytest.mark.parametrize("shape,flat", [((34161, 168), False), ((3416, 168), True), ((160006, 140), True), ((18000, 280), False),
+                                        ((1500, 280), True), ((60000, 260), True), ((2017, 2280), False), ((300, 2280), True),
+                                        ((3000, 1028), True), ((8000, 2280), True), ((8000, 2560), False)])
+def test_flat_form_against_the_space_moved(shape, flat):
+    """CPU: idle lanes count for less where the operands (4 bytes: one read and two written) move 16 MB or more."""
+    types = {n: "f32" for n in "abcyz"}
+    ptrs = {n: 0x100000 * (i + 1) for i, n in enumerate("abcyz")}
+    prog = _program(shape, ("dense", "column", "row"))[0]
+    assert ("ldf<0, 'u'>(a.in" in elementwise_source(prog, ptrs, types)) == flat
 
 
 @pytest.mark.gpu
