@@ -26,6 +26,23 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_b2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_b2 __attribute__((ext_vector_type(2), aligned(2)));
 
+// 8 consecutive 16-bit elements at s + k, zero at and past K: read where a row's last 8 lie (K >= 8; the
+// elements before k are shifted out), with no branch, so that a lane's tail loads stay in flight
+// together.
+__device__ __forceinline__ u32x4 load_tail8(const uint16_t* s, int64_t k, int64_t K) {
+  const int64_t over = k + 8 - K;  // elements past K
+  const int d = over <= 0 ? 0 : over >= 8 ? 8 : static_cast<int>(over);
+  const u32x4 v = *reinterpret_cast<const u32x4_b2*>(s + (over <= 0 ? k : K - 8));
+  uint64_t lo = v[0] | (static_cast<uint64_t>(v[1]) << 32), hi = v[2] | (static_cast<uint64_t>(v[3]) << 32);
+  if (d & 4) lo = hi, hi = 0;
+  const int sh = 16 * (d & 3);
+  lo = sh ? (lo >> sh) | (hi << (64 - sh)) : lo;
+  hi >>= sh;
+  if (d == 8) lo = 0, hi = 0;
+  return u32x4{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
+               static_cast<uint32_t>(hi >> 32)};
+}
+
 // ---------------------------------------------------------------- 16-bit floats
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
   return __uint_as_float(static_cast<uint32_t>(b) << 16);

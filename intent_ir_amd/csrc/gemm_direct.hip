@@ -62,23 +62,6 @@ __device__ __forceinline__ void load_cols(const uint16_t* p, uint32_t* d) {
   }
 }
 
-// 8 consecutive bf16 at s + k, zero at and past K: read where a row's last 8 lie (K >= 8; the
-// elements before k are shifted out), with no branch, so that a lane's tail loads stay in flight
-// together.
-__device__ __forceinline__ u32x4 load_tail8(const uint16_t* s, int64_t k, int64_t K) {
-  const int64_t over = k + 8 - K;  // elements past K
-  const int d = over <= 0 ? 0 : over >= 8 ? 8 : static_cast<int>(over);
-  const u32x4 v = *reinterpret_cast<const u32x4_b2*>(s + (over <= 0 ? k : K - 8));
-  uint64_t lo = v[0] | (static_cast<uint64_t>(v[1]) << 32), hi = v[2] | (static_cast<uint64_t>(v[3]) << 32);
-  if (d & 4) lo = hi, hi = 0;
-  const int sh = 16 * (d & 3);
-  lo = sh ? (lo >> sh) | (hi << (64 - sh)) : lo;
-  hi >>= sh;
-  if (d == 8) lo = 0, hi = 0;
-  return u32x4{static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi),
-               static_cast<uint32_t>(hi >> 32)};
-}
-
 template <int MF, int NF, bool kNT>
 struct Direct {
   static constexpr int KS = 64;                            // k per slab

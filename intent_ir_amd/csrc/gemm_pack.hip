@@ -127,21 +127,22 @@ bool shape_packs_a(int64_t M, int64_t K, bool ta) { return K % 8 != 0 || (ta && 
 bool shape_packs_b(int64_t N, int64_t K, bool tb) { return K % 8 != 0 || (!tb && N % 8 != 0); }
 
 // dst [R, K8] from a K-contiguous src [R, K] (leading dimension K): 16 bytes per thread, read at
-// the row's own 2-byte boundary.
+// the row's own 2-byte boundary, the end of a row without a branch (its elements one by one made
+// 2 x 7287 x 118 9.2 -> 9.7 us against the 4-byte loads of even rows before).
 __global__ __launch_bounds__(256) void pack_rows_kc(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
                                                     int64_t R, int64_t K, int64_t K8) {
   const int64_t chunks = K8 / 8;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= R * chunks) return;
   const int64_t r = t / chunks, k0 = (t % chunks) * 8;
-  const uint16_t* s = src + r * K + k0;
+  const uint16_t* s = src + r * K;
   u32x4 w = {0, 0, 0, 0};
-  if (k0 + 8 <= K) {
-    w = *reinterpret_cast<const u32x4_b2*>(s);
+  if (K >= 8) {
+    w = load_tail8(s, k0, K);
   } else {
 #pragma unroll
     for (int e = 0; e < 7; ++e)
-      if (k0 + e < K) w[e >> 1] |= static_cast<uint32_t>(s[e]) << (16 * (e & 1));
+      if (e < K) w[e >> 1] |= static_cast<uint32_t>(s[e]) << (16 * (e & 1));
   }
   *reinterpret_cast<u32x4*>(dst + r * K8 + k0) = w;
 }
