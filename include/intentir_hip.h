@@ -213,7 +213,7 @@ int64_t ihip_gemm_f32_workspace_size(int64_t M, int64_t N, int64_t K);
  * A is given as [K, M] and the product uses its transpose; when transpose_b, B is given as
  * [N, K].  Every layout runs the same MFMA schedule and accumulates in the same order, so a
  * transposed operand gives bit-identical C.  With B given as [N, K] the tiled kernel takes
- * any N (K % 8 == 0): C rows that are not 16-byte aligned are written with 2-byte stores. */
+ * any N (K % 8 == 0): C rows that are not 16-byte aligned are stored 16 bytes at a time too. */
 int ihip_gemm_bf16_bias_relu_t(const uint16_t* A, const uint16_t* B, const float* bias, uint16_t* C, int64_t M,
                                int64_t N, int64_t K, int transpose_a, int transpose_b, int relu, void* stream);
 
@@ -247,7 +247,7 @@ int64_t ihip_gemm_workspace_size(int64_t M, int64_t N, int64_t K, int transpose_
  * long; NULL / 0 allowed):
  *  - operands the tiled kernel cannot read in place are copied into it as K-contiguous rows
  *    of K rounded up to 8 elements (zeros past K) and the tiled kernel runs on the copies;
- *    C rows that are not 16-byte aligned are written with 2-byte stores.  Unsplit, results
+ *    C rows that are not 16-byte aligned are stored 16 bytes at a time too.  Unsplit, results
  *    are bit-identical to the guarded kernel's (the same zeros in the same k slots, the same
  *    MFMA order), which runs when the workspace is too small for the copies;
  *  - a grid of too few tiles (ihip_gemm_workspace_size) is split along K: each segment's

@@ -779,7 +779,7 @@ def test_gemm_split_k(hip, M, N, K, splits, ta, tb):
 @pytest.mark.parametrize("M,N,K", [(1000, 1001, 4096), (64, 3, 8192), (200, 4097, 4096)])
 def test_gemm_split_k_odd_n_with_b_as_nk(hip, M, N, K):
     """With B given as [N, K] any N runs in place; the partial rows are padded to a multiple of
-    4 floats and the reduce writes C with 2-byte stores where a row is not 8-byte aligned."""
+    4 floats and the reduce stores C 8 bytes at a time at any 2-byte boundary."""
     w = WORKLOADS["matmul"]
     b = {"M": M, "N": N, "K": K}
     inp = w.gen(b, seed=M + N + K, sigma=1.0)

@@ -263,7 +263,7 @@ def test_gemm_launch_descriptor_follows_the_fast_path(M, N, K, tile, path):
                                           (50257, False, 163840, "ihip_gemm_bf16_bias_relu_ws")])
 def test_gemm_odd_n_takes_the_tiled_kernel_with_b_as_nk(N, tb, lds, kid):
     """With B given as [N, K] (transpose_b) the rows of A and B stay 16-byte aligned at any N,
-    so the tiled kernel runs (C written with 2-byte stores); B as [K, N] with N % 8 != 0 is
+    so the tiled kernel runs (C stored at 2-byte boundaries); B as [K, N] with N % 8 != 0 is
     packed into a workspace as [N, K] first."""
     ir = matmul_bias_relu2d_ir()
     if tb:
