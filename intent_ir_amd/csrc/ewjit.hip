@@ -1103,10 +1103,16 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
   // whole lines, whose pieces two workgroups share, [8192, 4100] 63.2 -> 86.3, 65.8 -> 87.3, [524288, 33]
   // 48.3 -> 69.8, 48.8 -> 72.4; up to 256 MB [8192, 1024] 13.6 -> 15.4, 16.1 -> 17.0, [131072, 64] 11.7
   // -> 16.4, 15.6 -> 16.9.
-  // Vectors of 32-bit staged inputs are read past the caches ('v'), but with ordinary loads ('V') for rows
-  // of at most 32 elements while they and the outputs fit the 256 MB memory-side cache together, where
-  // that gained over the same buffers and over four sets ([493444, 17] 27.0 -> 22.6, 27.4 -> 23.7; [524288, 32] 26.0 -> 23.8,
-  // 27.5 -> 25.6); longer rows lose over rotating buffers ([98304, 256] 38.7 -> 32.4 but 39.4 -> 42.9).
+  // Vectors of 32-bit staged inputs are read past the caches ('v'), but with ordinary loads ('V'), which
+  // leave in the 256 MB memory-side cache what the next pass or an earlier kernel's reader finds, where
+  // that does not cost passes over rotating buffers (600 MB of them): 128 x 32 tiles up to 256 MB
+  // ([493444, 17] over the same buffers 27.0 -> 22.6, four sets 27.4 -> 23.7; [524288, 32] 26.0 -> 23.8, 27.5
+  // -> 25.6), and, where every operand is 4 bytes wide, 64 x 64 tiles of 64 to 100 MB with rows off 16-byte
+  // alignment ([86872, 143] 38.6 -> 32.1, rotating 39.7 -> 39.8; [296880, 34] 31.9 -> 24.5, 33.4 -> 33.5) or
+  // 80 (48 for rows that are not whole lines) to 160 MB with rows of at most 300 elements ([42668, 296]
+  // 24.1 -> 21.5, 27.3 -> 24.3; [108024, 76] 19.2 -> 17.7, 24.1 -> 23.1).  Elsewhere one side loses:
+  // [98304, 256] (201 MB) 38.7 -> 32.4 but 39.4 -> 42.9, [8192, 1024] 13.6 -> 15.7, ragged rows of 16 to 48
+  // MB up to 8% over rotating buffers, of 120 MB and more 3% over three sets.
   bool four = true, lines = shape[3] % 32 == 0;
   for (int k = 0; k < n_inputs; ++k) four &= esize(in_dt[k]) == 4 && (!((tile_mask >> k) & 1u) || stage_vec(k));
   for (int k = 0; k < n_outputs; ++k) {
@@ -1117,9 +1123,13 @@ bool plan_jit(const ihip_ew_instr* code, int n_code, const ihip_ew_operand* inpu
   int64_t tiled_bytes = 0;
   for (int k = 0; k < n_inputs; ++k) tiled_bytes += ((tile_mask >> k) & 1u) ? esize(in_dt[k]) : 0;
   for (int k = 0; k < n_outputs; ++k) tiled_bytes += esize(out_dt[k]);
-  const bool cached = tiled_bytes * a.rows * shape[3] <= int64_t(256) * 1000 * 1000;
+  const int64_t moved = tiled_bytes * a.rows * shape[3];
+  const bool cached = moved <= int64_t(256) * 1000 * 1000;
   f.wide = tile_mask != 0 && four && shape[2] > 64 && (shape[3] <= 32 || (lines && !cached));
-  const auto stage_kind = [&](int k) { return !stage_vec(k) ? 't' : f.wide && cached ? 'V' : 'v'; };
+  const int64_t least = shape[3] % 4 != 0 ? 64 : shape[3] > 300 ? 256 : shape[3] % 32 != 0 ? 48 : 80;  // MB
+  const int64_t most = shape[3] % 4 != 0 ? 100 : 160;
+  const bool ordinary = f.wide ? cached : four && moved >= least * 1000000 && moved <= most * 1000000;
+  const auto stage_kind = [&](int k) { return !stage_vec(k) ? 't' : ordinary ? 'V' : 'v'; };
   char(&in_kind)[IHIP_EW_NATIVE_MAX_INPUTS + 1] = f.in_kind;
   char(&out_kind)[IHIP_EW_NATIVE_MAX_OUTPUTS + 1] = f.out_kind;
   for (int k = 0; k < n_inputs; ++k) {

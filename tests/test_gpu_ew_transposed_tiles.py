@@ -45,6 +45,19 @@ def test_tile_extents_follow_types_and_shape(shape, wide):
         assert ("ld4c<0>(p" in src or "ld4c<4>(p" in src) == (took and small)
 
 
+@pytest.mark.parametrize("shape,ordinary", [((1, 86872, 143), True), ((1, 42668, 296), True), ((1, 108024, 76), True),
+                                            ((1, 86873, 143), False), ((1, 40000, 143), False), ((1, 4096, 4100), False),
+                                            ((1, 60000, 96), False), ((1, 117052, 128), True), ((1, 98304, 256), False),
+                                            ((1, 100000, 143), False), ((2, 43436, 143), True)])
+def test_staging_loads_of_64_x_64_tiles(shape, ordinary):
+    """CPU: ordinary loads where they cost rotating buffers nothing; 4-byte operands only."""
+    ptrs = {n: 0x100000 * (i + 1) for i, n in enumerate("abcy")}
+    for types in TYPES[:3]:
+        src = elementwise_source(_program(shape), ptrs, dict(zip("abcy", types)))
+        assert "#define EW_T2 64" in src
+        assert ("ld4c<" in src.split("ihip_ew_jit")[1]) == (ordinary and types[0] != "bf16")
+
+
 @pytest.mark.parametrize("shape,wide", LARGE)
 def test_wide_tiles_need_output_lines_of_their_own(shape, wide):
     """CPU: an output off a 128-byte boundary shares its lines between tiles; short rows do not mind."""
@@ -56,7 +69,8 @@ def test_wide_tiles_need_output_lines_of_their_own(shape, wide):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("types", TYPES)
-@pytest.mark.parametrize("shape", [s for s, _ in SHAPES] + [(1, 5800, 5888), (1, 8192, 4128), (1, 1048576, 32)])
+@pytest.mark.parametrize("shape", [s for s, _ in SHAPES] + [(1, 5800, 5888), (1, 8192, 4128), (1, 1048576, 32),
+                                                             (1, 60000, 143), (1, 42668, 296)])
 def test_tiled_form_equals_the_interpreter_kernel(hip, shape, types):
     import torch
 
